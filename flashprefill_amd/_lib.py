@@ -31,6 +31,7 @@ EXPORTS = (
     "fp_workspace_layout", "fp_workspace_bytes", "fp_flashprefill", "fp_plan", "fp_pool_k",
     "fp_search", "fp_select", "fp_sparse_attn_fwd", "fp_read_status", "fp_last_error",
     "fp_abi_version", "fp_flashprefill_noalloc", "fp_kv_cache_write", "fp_rope_qk",
+    "fp_paged_attention", "fp_paged_workspace_bytes",
 )
 NOALLOC_SCRATCH_BYTES = 96 * 1024 * 1024
 
@@ -102,6 +103,26 @@ class FpKvCacheArgs(ctypes.Structure):
     ]
 
 
+class FpPagedArgs(ctypes.Structure):
+    _fields_ = [
+        ("q", ctypes.c_void_p), ("q_stride_tok", ctypes.c_int64), ("q_stride_head", ctypes.c_int64),
+        ("o", ctypes.c_void_p), ("o_stride_tok", ctypes.c_int64), ("o_stride_head", ctypes.c_int64),
+        ("key_cache", ctypes.c_void_p), ("value_cache", ctypes.c_void_p),
+        ("kc_stride_block", ctypes.c_int64), ("kc_stride_slot", ctypes.c_int64),
+        ("kc_stride_head", ctypes.c_int64),
+        ("vc_stride_block", ctypes.c_int64), ("vc_stride_slot", ctypes.c_int64),
+        ("vc_stride_head", ctypes.c_int64),
+        ("cu_seqlens", ctypes.c_void_p), ("seqused", ctypes.c_void_p),
+        ("block_table", ctypes.c_void_p), ("table_stride", ctypes.c_int64),
+        ("num_tokens", ctypes.c_int64), ("num_blocks", ctypes.c_int64),
+        ("batch", ctypes.c_int32), ("table_width", ctypes.c_int32), ("block_size", ctypes.c_int32),
+        ("num_q_heads", ctypes.c_int32), ("num_kv_heads", ctypes.c_int32),
+        ("head_dim", ctypes.c_int32), ("dtype", ctypes.c_int32),
+        ("cu_is64", ctypes.c_int32), ("used_is64", ctypes.c_int32), ("table_is64", ctypes.c_int32),
+        ("softmax_scale", ctypes.c_float),
+    ]
+
+
 _LIB = None
 
 
@@ -126,13 +147,16 @@ def load(path: Path = LIB_PATH) -> ctypes.CDLL:
     lib.fp_flashprefill_noalloc.argtypes = [P, vp]
     lib.fp_kv_cache_write.argtypes = [ctypes.POINTER(FpKvCacheArgs), vp]
     lib.fp_rope_qk.argtypes = [ctypes.POINTER(FpRopeArgs), vp]
+    lib.fp_paged_attention.argtypes = [ctypes.POINTER(FpPagedArgs), vp, vp]
+    lib.fp_paged_workspace_bytes.argtypes = [ctypes.POINTER(FpPagedArgs)]
+    lib.fp_paged_workspace_bytes.restype = ctypes.c_size_t
     lib.fp_search.argtypes = [P, vp, vp, vp, vp]
     lib.fp_select.argtypes = [P, vp, vp, vp, vp]
     lib.fp_read_status.argtypes = [P, vp, vp, ctypes.POINTER(ctypes.c_uint32)]
     lib.fp_last_error.restype = ctypes.c_char_p
     lib.fp_abi_version.restype = ctypes.c_int
     for name in EXPORTS:
-        if name not in ("fp_workspace_bytes", "fp_last_error", "fp_abi_version"):
+        if name not in ("fp_workspace_bytes", "fp_paged_workspace_bytes", "fp_last_error", "fp_abi_version"):
             getattr(lib, name).restype = ctypes.c_int
     if lib.fp_abi_version() != ABI_VERSION:
         raise RuntimeError(f"{path.name} ABI {lib.fp_abi_version()} != expected {ABI_VERSION}")

@@ -455,6 +455,68 @@ int scratch_on_current_device(void** out) {
   return FP_OK;
 }
 
+int paged_valid(const fp_paged_args* a) {
+  if (!a) return fail(FP_E_INVALID_ARG, "paged arguments are NULL");
+  if (a->dtype != FP_DTYPE_BF16 && a->dtype != FP_DTYPE_F16)
+    return fail(FP_E_UNSUPPORTED, "paged: dtype %d unsupported (bf16 or fp16)", a->dtype);
+  if (a->head_dim != 64 && a->head_dim != 128 && a->head_dim != 256)
+    return fail(FP_E_UNSUPPORTED, "paged: head_dim %d unsupported (64, 128 or 256)", a->head_dim);
+  if (a->num_q_heads < 1 || a->num_kv_heads < 1 || a->num_q_heads % a->num_kv_heads)
+    return fail(FP_E_INVALID_ARG, "paged: num_q_heads (%d) must be a positive multiple of "
+                "num_kv_heads (%d)", a->num_q_heads, a->num_kv_heads);
+  if (a->num_tokens < 0 || a->num_blocks < 1 || a->batch < 1 || a->block_size < 1 ||
+      a->table_width < 0 || a->table_stride < 0)
+    return fail(FP_E_INVALID_ARG, "paged: sizes out of range");
+  if (a->num_tokens == 0) return FP_OK;
+  if (!a->q || !a->o || !a->key_cache || !a->value_cache || !a->cu_seqlens || !a->seqused ||
+      (!a->block_table && a->table_width > 0))
+    return fail(FP_E_INVALID_ARG, "paged: NULL pointer");
+  if (!aligned16(a->q) || !aligned16(a->o) || !aligned16(a->key_cache) ||
+      !aligned16(a->value_cache))
+    return fail(FP_E_INVALID_ARG, "paged: q, o and the caches must be 16-byte aligned");
+  const int64_t st[10] = {a->q_stride_tok,    a->q_stride_head,  a->o_stride_tok,
+                          a->o_stride_head,   a->kc_stride_block, a->kc_stride_slot,
+                          a->kc_stride_head,  a->vc_stride_block, a->vc_stride_slot,
+                          a->vc_stride_head};
+  for (int i = 0; i < 10; ++i)
+    if (st[i] < 0 || st[i] % 8)
+      return fail(FP_E_INVALID_ARG, "paged: strides must be non-negative multiples of 8 elements");
+  // a lane's offset inside a page (16 slots) is formed in 32 bits
+  if (a->kc_stride_slot >= (int64_t(1) << 24) || a->vc_stride_slot >= (int64_t(1) << 24))
+    return fail(FP_E_UNSUPPORTED, "paged: slot strides of 2^24 elements or more");
+  // key positions, and query rows x heads (the merge's grid), are 32-bit
+  if (static_cast<int64_t>(a->table_width) * a->block_size >= (int64_t(1) << 30))
+    return fail(FP_E_UNSUPPORTED, "paged: 2^30 or more tokens per sequence");
+  if (a->num_tokens * a->num_q_heads >= (int64_t(1) << 30))
+    return fail(FP_E_UNSUPPORTED, "paged: 2^30 or more query rows");
+  return FP_OK;
+}
+
+// Row tiles and chunk slots of a paged call. Tiles: 16 rows (query tokens x
+// the query heads of a KV head) of one sequence; at most T G / 16 + B of them,
+// and no more than each token's rows on their own would make. Chunk slots:
+// about kTarget workgroups in all (several rounds of the card's ~768 resident
+// ones, so that sequences of different lengths balance), no more than
+// kPagedMaxChunks, and none shorter than kPagedMinChunk keys.
+struct PagedSplit {
+  int64_t tiles;
+  int nc;
+  size_t bytes;
+};
+PagedSplit paged_split(const fp_paged_args* a) {
+  constexpr int64_t kTarget = 8192;
+  PagedSplit r;
+  const int64_t G = a->num_q_heads / a->num_kv_heads, T = a->num_tokens;
+  r.tiles = std::min<int64_t>(T * ((G + 15) / 16), T * G / 16 + a->batch);
+  const int64_t longest = static_cast<int64_t>(a->table_width) * a->block_size;
+  const int64_t wgs = std::max<int64_t>(1, r.tiles * a->num_kv_heads);
+  int64_t nc = std::min<int64_t>(fp::kPagedMaxChunks, (kTarget + wgs - 1) / wgs);
+  nc = std::min<int64_t>(nc, (longest + fp::kPagedMinChunk - 1) / fp::kPagedMinChunk);
+  r.nc = static_cast<int>(std::max<int64_t>(1, nc));
+  r.bytes = r.nc > 1 ? static_cast<size_t>(T * a->num_q_heads * r.nc) * (a->head_dim + 2) * 4 : 0;
+  return r;
+}
+
 }  // namespace
 
 extern "C" {
@@ -579,6 +641,60 @@ int fp_rope_qk(const fp_rope_args* a, void* stream) {
   r.eps = a->eps;
   const hipError_t e = fp::launch_rope(r, a->dtype, static_cast<hipStream_t>(stream));
   return e == hipSuccess ? FP_OK : hip_fail(e, "rope launch");
+}
+
+size_t fp_paged_workspace_bytes(const fp_paged_args* a) {
+  return paged_valid(a) == FP_OK ? paged_split(a).bytes : 0;
+}
+
+int fp_paged_attention(const fp_paged_args* a, void* ws, void* stream) {
+  const int rc = paged_valid(a);
+  if (rc != FP_OK) return rc;
+  if (a->num_tokens == 0) return FP_OK;
+  const PagedSplit sp = paged_split(a);
+  if (sp.bytes > 0 && !ws) return fail(FP_E_INVALID_ARG, "paged: workspace is NULL");
+  if (!aligned16(ws)) return fail(FP_E_INVALID_ARG, "paged: workspace must be 16-byte aligned");
+  fp::PagedArgs r;
+  r.q = a->q;
+  r.o = a->o;
+  r.kc = a->key_cache;
+  r.vc = a->value_cache;
+  r.qst = a->q_stride_tok;
+  r.qhs = a->q_stride_head;
+  r.ost = a->o_stride_tok;
+  r.ohs = a->o_stride_head;
+  r.kcb = a->kc_stride_block;
+  r.kcs = a->kc_stride_slot;
+  r.kch = a->kc_stride_head;
+  r.vcb = a->vc_stride_block;
+  r.vcs = a->vc_stride_slot;
+  r.vch = a->vc_stride_head;
+  r.cu = a->cu_seqlens;
+  r.used = a->seqused;
+  r.table = a->block_table;
+  r.cu64 = a->cu_is64;
+  r.used64 = a->used_is64;
+  r.table64 = a->table_is64;
+  r.table_stride = a->table_stride;
+  r.T = a->num_tokens;
+  r.nblocks = a->num_blocks;
+  r.B = a->batch;
+  r.width = a->table_width;
+  r.bs = a->block_size;
+  r.bs_shift = -1;
+  for (int sh = 0; sh < 31; ++sh)
+    if ((1 << sh) == a->block_size) r.bs_shift = sh;
+  r.Hq = a->num_q_heads;
+  r.Hkv = a->num_kv_heads;
+  r.G = a->num_q_heads / a->num_kv_heads;
+  r.scale_log2 = a->softmax_scale * static_cast<float>(1.4426950408889634);
+  r.nc = sp.nc;
+  r.part = static_cast<float*>(ws);
+  r.ml = sp.nc > 1 ? static_cast<float*>(ws) + a->num_tokens * a->num_q_heads * sp.nc * a->head_dim
+                   : nullptr;
+  const hipError_t e = fp::launch_paged(r, a->dtype, a->head_dim, sp.tiles,
+                                        static_cast<hipStream_t>(stream));
+  return e == hipSuccess ? FP_OK : hip_fail(e, "paged attention launch");
 }
 
 int fp_kv_cache_write(const fp_kv_cache_args* a, void* stream) {

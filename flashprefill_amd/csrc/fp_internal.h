@@ -120,6 +120,32 @@ struct KvCacheArgs {
   int32_t elem_bytes;
 };
 
+// Attention over a paged cache (fp_paged.hip)
+constexpr int kPagedMinChunk = 256;  // keys per workgroup at least
+constexpr int kPagedMaxChunks = 128;  // chunk slots per query row at most (k_paged_merge)
+
+struct PagedArgs {
+  const void* q;
+  const void* kc;
+  const void* vc;
+  void* o;
+  int64_t qst, qhs, ost, ohs;
+  int64_t kcb, kcs, kch, vcb, vcs, vch;  // cache strides: block, slot, head
+  const void* cu;     // B + 1 query offsets
+  const void* used;   // B cached lengths
+  const void* table;  // B rows of `width` page numbers, table_stride apart
+  int32_t cu64, used64, table64;  // the arrays hold 64-bit integers
+  int64_t table_stride;
+  int64_t T;        // query rows
+  int64_t nblocks;  // pages of the cache
+  int32_t B, width, bs, bs_shift;  // bs_shift: log2(bs), -1 when bs is no power of two
+  int32_t Hq, Hkv, G;
+  float scale_log2;  // softmax scale * log2 e
+  int32_t nc;        // chunk slots per row
+  float* part;       // [T * Hq][nc][d] unnormalised outputs
+  float* ml;         // [T * Hq][nc] (m, l) pairs
+};
+
 struct RopeArgs {
   void* q;
   int64_t q_stride_tok, q_stride_head;
@@ -147,6 +173,7 @@ auto with_head_dim(int head_dim, F&& f) {
 
 hipError_t launch_plan(const PlanArgs& a, hipStream_t s);
 hipError_t launch_rope(const RopeArgs& a, int dtype, hipStream_t s);
+hipError_t launch_paged(const PagedArgs& a, int dtype, int head_dim, int64_t tiles, hipStream_t s);
 hipError_t launch_kv_cache_write(const KvCacheArgs& a, hipStream_t s);
 hipError_t launch_pool(const PoolArgs& a, int dtype, int head_dim, int64_t grid, hipStream_t s);
 // k_plan then k_pool as one launch (16-bit inputs, batch <= kSmallPlanBatch)

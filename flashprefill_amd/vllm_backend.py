@@ -42,6 +42,7 @@ import torch
 
 from . import _lib
 from .flashprefill_varlen_func import flash_prefill_varlen_func
+from .runtime import WORKSPACES
 
 # Per-model selection configs of the reference patch
 # (patches/patch_loader_vllm_0_12_0.py:13-40): block 128, sink 2, window 4,
@@ -103,13 +104,104 @@ def paged_decode_attention(query: torch.Tensor, key_cache: torch.Tensor,
                            value_cache: torch.Tensor, out: torch.Tensor,
                            cu_seqlens_q: torch.Tensor, seqused_k: torch.Tensor,
                            block_table: torch.Tensor, softmax_scale: float) -> None:
-    """Decode attention over the paged cache (the role of vLLM's
+    """Attention over the paged cache (the role of vLLM's
     ``flash_attn_varlen_func`` with a block table in the reference's decode
     branch): every query row of sequence b attends causally to the first
     ``seqused_k[b]`` cached tokens, the last query sitting at position
-    ``seqused_k[b] - 1``. torch GPU ops in fp32 (one small gather per
-    sequence); it is the default when no vLLM decode op is injected, not part
-    of the prefill path."""
+    ``seqused_k[b] - 1``; fp32 softmax and sums. The default when no vLLM
+    decode op is injected, not part of the prefill path.
+
+    bf16 / fp16 tensors on the GPU (head_dim 64, 128 or 256) take the HIP
+    kernels behind ``fp_paged_attention``: no host synchronisation, so what
+    only the device sees is checked there (a sequence with more cached tokens
+    than its table row has room for, or a page outside the cache, gets NaN
+    rows). Every other call (CPU, fp32, other head dims or layouts, inputs
+    that require gradients) takes the torch composition."""
+    if _paged_kernel_takes(query, key_cache, value_cache, out, cu_seqlens_q, seqused_k,
+                           block_table):
+        _paged_attention_kernel(query, key_cache, value_cache, out, cu_seqlens_q, seqused_k,
+                                block_table, softmax_scale)
+    else:
+        paged_attention_reference(query, key_cache, value_cache, out, cu_seqlens_q, seqused_k,
+                                  block_table, softmax_scale)
+
+
+_INDEX = (torch.int32, torch.int64)
+
+
+def _rows_ok(t: torch.Tensor) -> bool:
+    return (t.stride(-1) == 1 and t.data_ptr() % 16 == 0
+            and all(s % 8 == 0 and s >= 0 for s in t.stride()[:-1]))
+
+
+def _paged_kernel_takes(query, key_cache, value_cache, out, cu, used, table) -> bool:
+    """Whether the HIP kernels take this call as it is: 16-bit tensors of one
+    type on one GPU, head_dim 64 / 128 / 256, 16-byte aligned rows, int32 /
+    int64 metadata of matching shapes."""
+    if not query.is_cuda or query.dtype not in _DTYPES:
+        return False
+    dev, dt = query.device, query.dtype
+    if query.dim() != 3 or out.dim() != 3 or key_cache.dim() != 4 or \
+            value_cache.shape != key_cache.shape:
+        return False
+    nb, bs, hkv, d = key_cache.shape
+    T, hq, dq = query.shape
+    if d not in (64, 128, 256) or dq != d or nb < 1 or bs < 1 or hkv < 1 or hq < 1 or hq % hkv or \
+            out.shape[0] < T or out.shape[1:] != query.shape[1:]:
+        return False
+    for t in (query, key_cache, value_cache, out):
+        if t.dtype != dt or t.device != dev or not _rows_ok(t):
+            return False
+    if key_cache.stride(1) >= 1 << 24 or value_cache.stride(1) >= 1 << 24:
+        return False
+    if cu.dim() != 1 or used.dim() != 1 or table.dim() != 2 or cu.numel() < 2:
+        return False
+    B = cu.numel() - 1
+    if used.numel() < B or table.shape[0] < B or cu.dtype not in _INDEX or \
+            used.dtype not in _INDEX or table.dtype not in _INDEX:
+        return False
+    if table.shape[1] * bs >= 1 << 30 or T * hq >= 1 << 30:
+        return False
+    return not (torch.is_grad_enabled() and any(t.requires_grad for t in
+                                                (query, key_cache, value_cache, out)))
+
+
+def _paged_attention_kernel(query, key_cache, value_cache, out, cu, used, table, scale) -> None:
+    dev = query.device
+    nb, bs, hkv, d = key_cache.shape
+    T, hq = query.shape[:2]
+    cu, used = cu.to(dev).contiguous(), used.to(dev).contiguous()
+    table = table.to(dev)
+    if table.stride(1) != 1:
+        table = table.contiguous()
+    a = _lib.FpPagedArgs()
+    a.q, a.q_stride_tok, a.q_stride_head = query.data_ptr(), query.stride(0), query.stride(1)
+    a.o, a.o_stride_tok, a.o_stride_head = out.data_ptr(), out.stride(0), out.stride(1)
+    a.key_cache, a.value_cache = key_cache.data_ptr(), value_cache.data_ptr()
+    a.kc_stride_block, a.kc_stride_slot, a.kc_stride_head = key_cache.stride()[:3]
+    a.vc_stride_block, a.vc_stride_slot, a.vc_stride_head = value_cache.stride()[:3]
+    a.cu_seqlens, a.seqused, a.block_table = cu.data_ptr(), used.data_ptr(), table.data_ptr()
+    a.table_stride, a.num_tokens, a.num_blocks = table.stride(0), T, nb
+    a.batch, a.table_width, a.block_size = cu.numel() - 1, table.shape[1], bs
+    a.num_q_heads, a.num_kv_heads, a.head_dim = hq, hkv, d
+    a.dtype = _DTYPES[query.dtype]
+    a.cu_is64, a.used_is64 = cu.dtype == torch.int64, used.dtype == torch.int64
+    a.table_is64 = table.dtype == torch.int64
+    a.softmax_scale = float(scale)
+    lib = _lib.load()
+    with torch.cuda.device(dev):
+        ws = WORKSPACES.get(dev, max(int(lib.fp_paged_workspace_bytes(ctypes.byref(a))), 256))
+        _lib.check(lib.fp_paged_attention(ctypes.byref(a), ws.data_ptr(),
+                                          torch.cuda.current_stream(dev).cuda_stream))
+
+
+def paged_attention_reference(query: torch.Tensor, key_cache: torch.Tensor,
+                              value_cache: torch.Tensor, out: torch.Tensor,
+                              cu_seqlens_q: torch.Tensor, seqused_k: torch.Tensor,
+                              block_table: torch.Tensor, softmax_scale: float) -> None:
+    """The torch composition of ``paged_decode_attention`` in fp32 (one small
+    gather per sequence): the kernels' reference, and the path of the calls
+    they do not take."""
     cu = cu_seqlens_q.tolist()
     used = seqused_k.tolist()
     _, bs, hkv, d = key_cache.shape
@@ -138,7 +230,7 @@ def paged_decode_attention(query: torch.Tensor, key_cache: torch.Tensor,
 @dataclass
 class HookOps:
     """The operations the hooked forward calls; the defaults are this
-    package's (KV-cache write kernel, FlashPrefill, torch paged decode).
+    package's (KV-cache write kernel, FlashPrefill, paged attention).
     ``encoder`` and ``cascade`` take the impl and the reference's arguments
     and default to raising: they stay vLLM's."""
     cache_write: Callable[..., None] = reshape_and_cache

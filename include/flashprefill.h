@@ -199,6 +199,45 @@ typedef struct fp_kv_cache_args {
 } fp_kv_cache_args;
 int fp_kv_cache_write(const fp_kv_cache_args* a, void* stream);
 
+/* Attention over a paged KV cache (decode steps, and prefill whose prefix is
+ * cached): query rows cu[b] .. cu[b + 1] - 1 of sequence b are its last tokens,
+ * i.e. row t attends to the first used[b] - (cu[b + 1] - 1 - t) cached tokens,
+ * and query head h reads KV head h / (num_q_heads / num_kv_heads). Cached token
+ * k of sequence b is at page table[b][k / block_size], slot k % block_size.
+ * fp32 softmax and sums (the probabilities are not rounded to the input type).
+ * Replaces vLLM's flash_attn_varlen_func with a block table in the decode
+ * branch (patches/patch_loader_vllm_0_12_0.py:201-225,
+ * patch_loader_vllm_0_10_0.py:270-368). No host synchronisation: what the host
+ * cannot see is checked by the kernels. Offsets outside [0, num_tokens] or
+ * descending give the sequence no rows; more cached tokens than the table has
+ * room for, or a page number outside the cache, make its rows NaN; a row with
+ * no cached token to attend to is NaN, a sequence of no cached tokens 0.
+ * Strides in elements (multiples of 8, 16-byte aligned bases), head dim
+ * contiguous. The integer arrays hold 32- or 64-bit integers. */
+typedef struct fp_paged_args {
+    const void* q;            /* (num_tokens, num_q_heads, head_dim) */
+    int64_t q_stride_tok, q_stride_head;
+    void* o;                  /* as q */
+    int64_t o_stride_tok, o_stride_head;
+    const void* key_cache;    /* (num_blocks, block_size, num_kv_heads, head_dim) */
+    const void* value_cache;
+    int64_t kc_stride_block, kc_stride_slot, kc_stride_head;
+    int64_t vc_stride_block, vc_stride_slot, vc_stride_head;
+    const void* cu_seqlens;   /* device, batch + 1 entries */
+    const void* seqused;      /* device, batch entries */
+    const void* block_table;  /* device, batch rows of table_width entries */
+    int64_t table_stride;     /* entries between rows */
+    int64_t num_tokens;
+    int64_t num_blocks;
+    int32_t batch, table_width, block_size;
+    int32_t num_q_heads, num_kv_heads, head_dim; /* head_dim 64, 128 or 256 */
+    int32_t dtype;            /* FP_DTYPE_BF16 or FP_DTYPE_F16 */
+    int32_t cu_is64, used_is64, table_is64;
+    float softmax_scale;
+} fp_paged_args;
+size_t fp_paged_workspace_bytes(const fp_paged_args* a); /* 0: none needed, or invalid */
+int fp_paged_attention(const fp_paged_args* a, void* workspace, void* stream);
+
 /* Rotary position embedding (rotate-half) with optional per-head RMSNorm, in
  * place on the query and key heads of a decoder-layer attention block. No
  * kernel of the reference does this: it replaces the torch steps its model

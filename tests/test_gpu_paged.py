@@ -1,0 +1,164 @@
+"""Paged attention kernels (fp_paged_attention) against float64 attention over
+the gathered pages: decode and several queries per sequence, edges of the
+16-key tiles, of the 32- and 128-key rounds and of the chunks, page sizes that
+are and are not multiples of 16, head dims, GQA ratios, metadata types."""
+
+import math
+
+import pytest
+import torch
+
+from flashprefill_amd import vllm_backend as vb
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _case(lens, news, hq, hkv, d, page, dtype, seed=0, index=torch.int32, width=None, spare=3):
+    g = torch.Generator().manual_seed(seed)
+    per = [(n + page - 1) // page for n in lens]
+    total = sum(per) + spare
+    perm = torch.randperm(total, generator=g)
+    table = torch.full((len(lens), max(width or 0, max(per), 1)), -1, dtype=index)
+    at = 0
+    for b, m in enumerate(per):
+        table[b, :m] = perm[at:at + m].to(index)
+        at += m
+    # slots past a sequence's end hold NaN: they must never reach the output
+    kc = torch.full((total, page, hkv, d), float("nan"), dtype=dtype)
+    vc = torch.full((total, page, hkv, d), float("nan"), dtype=dtype)
+    for b, n in enumerate(lens):
+        for j in range(per[b]):
+            m = min(page, n - j * page)
+            kc[table[b, j], :m] = torch.randn(m, hkv, d, generator=g).to(dtype)
+            vc[table[b, j], :m] = torch.randn(m, hkv, d, generator=g).to(dtype)
+    q = (1.5 * torch.randn(sum(news), hq, d, generator=g)).to(dtype)
+    cu = torch.tensor([0] + list(torch.tensor(news).cumsum(0)), dtype=index)
+    used = torch.tensor(lens, dtype=index)
+    return q, kc, vc, cu, used, table
+
+
+def _want(q, kc, vc, cu, used, table, scale):
+    out = torch.zeros(q.shape, dtype=torch.float64)
+    hq, hkv, page = q.shape[1], kc.shape[2], kc.shape[1]
+    for b in range(used.numel()):
+        n, q0, q1 = int(used[b]), int(cu[b]), int(cu[b + 1])
+        if n == 0:
+            continue
+        rows = table[b, :(n + page - 1) // page].long()
+        k = kc[rows].reshape(-1, hkv, q.shape[2])[:n].double().repeat_interleave(hq // hkv, 1)
+        v = vc[rows].reshape(-1, hkv, q.shape[2])[:n].double().repeat_interleave(hq // hkv, 1)
+        s = torch.einsum("qhd,khd->hqk", q[q0:q1].double(), k) * scale
+        pos = torch.arange(n - (q1 - q0), n).view(1, -1, 1)
+        s = s.masked_fill(torch.arange(n).view(1, 1, -1) > pos, float("-inf"))
+        out[q0:q1] = torch.einsum("hqk,khd->qhd", torch.softmax(s, -1), v)
+    return out
+
+
+def _run(args, scale):
+    dev = [t.to(DEV) for t in args]
+    out = torch.full(args[0].shape, 7.0, dtype=args[0].dtype, device=DEV)
+    assert vb._paged_kernel_takes(dev[0], dev[1], dev[2], out, *dev[3:])
+    vb.paged_decode_attention(dev[0], dev[1], dev[2], out, *dev[3:], scale)
+    return out.cpu()
+
+
+def _check(args, scale):
+    got, want = _run(args, scale).double(), _want(*args, scale)
+    # the output is rounded once to the input type: half a spacing, i.e. 2^-8
+    # (bf16, 8-bit significand) or 2^-11 (fp16, 11-bit) of the value at most;
+    # the fp32 scores, sums and exp2 before it add a few 2^-24 of |v| ~ 4
+    eps = 2.0 ** -8 if args[0].dtype == torch.bfloat16 else 2.0 ** -11
+    bound = want.abs() * eps * 1.01 + 2e-6
+    nan = want.isnan()
+    assert torch.equal(got.isnan(), nan)
+    assert ((got - want).abs()[~nan] <= bound[~nan]).all(), (got - want)[~nan].abs().max()
+
+
+@pytest.mark.parametrize("lens", [[1, 15, 16, 17], [31, 32, 33, 127], [128, 129, 255, 256],
+                                  [257, 384, 511, 640], [3000, 1, 40, 700]])
+@pytest.mark.parametrize("hq,hkv,d,dtype", [(32, 8, 128, torch.bfloat16), (28, 4, 128, torch.float16),
+                                            (8, 8, 64, torch.float16), (40, 2, 64, torch.bfloat16),
+                                            (8, 2, 256, torch.bfloat16), (6, 3, 256, torch.float16)])
+def test_decode(lens, hq, hkv, d, dtype):
+    _check(_case(lens, [1] * len(lens), hq, hkv, d, 16, dtype), 1 / math.sqrt(d))
+
+
+@pytest.mark.parametrize("page", [1, 5, 16, 24, 32, 48, 256])
+@pytest.mark.parametrize("index", [torch.int32, torch.int64])
+def test_page_sizes_and_index_types(page, index):
+    _check(_case([700, 33, 260], [1, 2, 1], 8, 2, 128, page, torch.bfloat16, index=index),
+           1 / math.sqrt(128))
+
+
+@pytest.mark.parametrize("lens,news", [([40, 300, 2100], [1, 7, 33]), ([5, 600, 64], [5, 0, 64]),
+                                       ([900, 0, 1300], [200, 3, 130]), ([3, 50], [6, 1]),
+                                       ([1500], [700])])
+@pytest.mark.parametrize("hq,hkv,d,dtype", [(28, 4, 128, torch.bfloat16), (8, 8, 64, torch.float16),
+                                            (8, 2, 256, torch.bfloat16), (32, 8, 128, torch.float16),
+                                            (4, 1, 64, torch.bfloat16), (4, 2, 256, torch.float16)])
+def test_several_queries(lens, news, hq, hkv, d, dtype):
+    # [3, 50] / [6, 1]: rows before the first cached token see nothing (NaN, as
+    # softmax over no key); a sequence of no cached tokens gives 0
+    _check(_case(lens, news, hq, hkv, d, 16, dtype), 1 / math.sqrt(d))
+
+
+def test_wide_table_and_many_sequences():
+    # a table far wider than the sequences (a server's limit), and more
+    # sequences than one round of the tile search covers
+    _check(_case([100, 2000], [1, 1], 8, 2, 128, 16, torch.bfloat16, width=4096), 0.08)
+    lens = [(37 * i) % 300 + 1 for i in range(150)]
+    _check(_case(lens, [1 + (i % 3 == 0) for i in range(150)], 4, 2, 64, 16, torch.bfloat16), 0.125)
+
+
+def test_one_long_sequence_uses_every_chunk_slot():
+    _check(_case([40000], [1], 4, 1, 128, 16, torch.bfloat16), 0.09)
+
+
+def test_strided_inputs_and_untouched_rows():
+    q, kc, vc, cu, used, table = _case([300, 70], [1, 1], 8, 2, 128, 16, torch.bfloat16)
+    T = 5
+    qkv = torch.zeros(T, 12, 128, dtype=torch.bfloat16)
+    qkv[:2, 2:10] = q
+    qd = qkv.to(DEV)[:, 2:10]
+    out = torch.full((T, 8, 128), 7.0, dtype=torch.bfloat16, device=DEV)
+    vb.paged_decode_attention(qd, kc.to(DEV), vc.to(DEV), out, cu.to(DEV), used.to(DEV),
+                              table.to(DEV), 0.1)
+    want = _run((q, kc, vc, cu, used, table), 0.1)
+    assert torch.equal(out[:2].cpu(), want)
+    assert (out[2:] == 7.0).all()
+
+
+def test_what_only_the_device_sees():
+    # a length beyond the table and a page outside the cache: NaN rows, the
+    # other sequences as they are; no access outside the cache
+    q, kc, vc, cu, used, table = _case([300, 70, 40], [1, 1, 1], 8, 2, 128, 16, torch.bfloat16)
+    want = _run((q, kc, vc, cu, used, table), 0.1)
+    u2 = used.clone()
+    u2[0] = table.shape[1] * 16 + 1
+    t2 = table.clone()
+    t2[2, 1] = kc.shape[0]
+    got = _run((q, kc, vc, cu, u2, t2), 0.1)
+    assert got[0].isnan().all() and got[2].isnan().all()
+    assert torch.equal(got[1], want[1])
+
+
+def test_capture_and_replay():
+    q, kc, vc, cu, used, table = [t.to(DEV) for t in
+                                  _case([900, 70], [1, 1], 8, 2, 128, 16, torch.bfloat16)]
+    out = torch.zeros_like(q)
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        vb.paged_decode_attention(q, kc, vc, out, cu, used, table, 0.1)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        vb.paged_decode_attention(q, kc, vc, out, cu, used, table, 0.1)
+    for n in (900, 300, 897):
+        used[0] = n
+        want = torch.zeros_like(q)
+        vb.paged_decode_attention(q, kc, vc, want, cu, used, table, 0.1)
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
