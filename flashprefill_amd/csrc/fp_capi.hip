@@ -107,6 +107,35 @@ int validate(const fp_problem* p) {
   return FP_OK;
 }
 
+// Chunk slots per row of the fp32 attention and list entries per chunk. A
+// problem of few rows would wait for its longest one (the card runs two
+// workgroups per CU, 512 at once), and unlike the 16-bit split rows any row may
+// be dense here, so every row gets 1536 / rows slots: 4K tokens x 8 heads, 256
+// rows, d = 64: attention 169 us with 2 slots, 101 with 4, 98 with 6, 109 with
+// 7 (more partials). From 769 rows on there is one slot. The partials are
+// held to kF32PartialBytes and, with the rest of the workspace (`base` bytes),
+// to the static scratch of fp_flashprefill_noalloc, so that no problem outgrows
+// it for their sake.
+struct F32Split {
+  int chunks, blocks;
+  size_t bytes;
+};
+F32Split f32_split(const fp_problem* p, int64_t nb_max, int64_t cap, size_t base) {
+  constexpr int64_t kSlots = 1536;
+  constexpr size_t kF32PartialBytes = size_t(64) << 20;
+  F32Split r = {1, static_cast<int>(nb_max), 0};
+  if (p->dtype != FP_DTYPE_F32) return r;
+  const int64_t blk = plan_block(p), rows = p->num_q_heads * cap;
+  const size_t per = static_cast<size_t>(rows) * 4 * (blk * p->head_dim + 2 * blk);
+  int64_t n = std::min<int64_t>({fp::kF32MaxChunks, kSlots / rows, nb_max});
+  n = std::min<int64_t>(n, kF32PartialBytes / per);
+  if (n < 2 || base + n * per + 512 > FP_NOALLOC_SCRATCH_BYTES) return r;
+  r.chunks = static_cast<int>(n);
+  r.blocks = static_cast<int>((nb_max + n - 1) / n);
+  r.bytes = n * per;
+  return r;
+}
+
 int layout(const fp_problem* p, fp_ws_layout* L) {
   const int rc = validate(p);
   if (rc != FP_OK) return rc;
@@ -187,7 +216,9 @@ int layout(const fp_problem* p, fp_ws_layout* L) {
   // units region: count and queue words, the unit records, then one arrival
   // counter per (head, unit) for the split rows merged inside the attention
   L->units_off = off;      off = align_up(off + 64 + sizeof(fp::UnitRec) * units + 4 * Hq * units);
-  L->part_off = off;       off = align_up(off + 4 * Hq * units * (blk * d + 2 * blk));
+  L->part_off = off;
+  off = align_up(off + (p->dtype == FP_DTYPE_F32 ? f32_split(p, nb_max, cap, off).bytes
+                                                 : 4 * Hq * units * (blk * d + 2 * blk)));
   L->total_bytes = off;
   return FP_OK;
 }
@@ -399,8 +430,14 @@ int run_attn(const fp_problem* p, const fp_ws_layout& L, void* ws, hipStream_t s
   a.ratio = block_ratio(p);
   const int blk = plan_block(p);
   hipError_t e;
+  a.f32_chunks = 1;
+  a.f32_chunk_blocks = L.nb_max;
   if (p->dtype == FP_DTYPE_F32) {
-    e = fp::launch_attn_f32(a, p->head_dim, blk, a.total_slots, s);
+    const F32Split sp = f32_split(p, L.nb_max, L.nb_sum_cap, L.part_off);
+    a.f32_chunks = sp.chunks;
+    a.f32_chunk_blocks = sp.blocks;
+    a.total_slots *= sp.chunks;
+    e = fp::launch_attn_f32(a, p->head_dim, blk, s);
   } else {
     // Persistent grid (every resident workgroup loops over its XCD's queue)
     // once there are at least 4 slots per resident workgroup: it saves the

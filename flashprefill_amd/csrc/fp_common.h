@@ -16,6 +16,7 @@ constexpr int kMaxBlocks = 8192;  // blocks per sequence (1,048,576 tokens at bl
 constexpr int kSmallPlanBatch = 16;  // batches planned inside the pooling launch (k_plan_pool)
 constexpr int kMaxChunks = 8;        // chunks of one split row (host policy, k_merge)
 constexpr int kMaxInlineChunks = 8;  // chunks merged inside the attention kernel
+constexpr int kF32MaxChunks = 8;     // chunk slots of a row, fp32 inputs (k_merge_f32)
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));

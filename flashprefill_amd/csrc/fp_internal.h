@@ -101,6 +101,10 @@ struct AttnArgs {
   int32_t* arrivals;
   int32_t merge_inline;
   int32_t ratio;  // > 1: row records are indexed by tile (block_size 256)
+  // fp32 inputs: chunk slots per row and list entries per chunk (k_attn_f32);
+  // part then holds [Hq][nb_sum_cap (by tile)][f32_chunks] partials
+  int32_t f32_chunks;
+  int32_t f32_chunk_blocks;
 };
 
 struct KvCacheArgs {
@@ -185,7 +189,6 @@ hipError_t launch_attn(const AttnArgs& a, int dtype, int head_dim, int block, in
                        bool persist, hipStream_t s);
 // combines the chunk partials of the split rows into their output rows
 hipError_t launch_merge(const AttnArgs& a, int dtype, int head_dim, int block, hipStream_t s);
-hipError_t launch_attn_f32(const AttnArgs& a, int head_dim, int block, int64_t grid,
-                           hipStream_t s);
+hipError_t launch_attn_f32(const AttnArgs& a, int head_dim, int block, hipStream_t s);
 
 }  // namespace fp

@@ -1,0 +1,109 @@
+"""fp32 attention on three-part bf16 products: error against float64 over
+magnitudes, rows in one and in several chunk slots, and the values that do not
+go through the split (2^56 and above, infinities, NaN)."""
+
+import math
+
+import pytest
+import torch
+
+from flashprefill_amd import flash_prefill, flash_prefill_varlen_func
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _dense(q, k, v):
+    """causal attention in float64, q (S, Hq, d)"""
+    S, hq, d = q.shape
+    g = hq // k.shape[1]
+    q, k, v = [t.double().permute(1, 0, 2) for t in (q, k, v)]
+    k, v = k.repeat_interleave(g, 0), v.repeat_interleave(g, 0)
+    s = torch.matmul(q, k.transpose(1, 2).contiguous()) / math.sqrt(d)
+    s = s.masked_fill(torch.ones(S, S, dtype=torch.bool, device=q.device).triu(1), -math.inf)
+    return torch.matmul(torch.softmax(s, -1), v).permute(1, 0, 2)
+
+
+def _run(q, k, v, block=128):
+    o = torch.empty_like(q)
+    cu = torch.tensor([0, q.shape[0]], dtype=torch.int32, device=DEV)
+    flash_prefill_varlen_func(q, k, v, o, cu, q.shape[0], 0.0, block)  # alpha 0: every block
+    return o
+
+
+@pytest.mark.parametrize("block", [64, 128])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("S,hq,hkv", [(1, 2, 1), (129, 2, 1), (700, 4, 2), (2100, 2, 2),
+                                      (1023, 24, 8)])
+@pytest.mark.parametrize("kscale,vscale", [(1.0, 1.0), (1e-3, 1e6), (30.0, 1e-12)])
+def test_error_against_float64(block, d, S, hq, hkv, kscale, vscale):
+    # 2 heads: several chunk slots per row; (1023, 24): one or two
+    g = torch.Generator(device=DEV).manual_seed(S + d)
+    q = torch.randn(S, hq, d, generator=g, device=DEV)
+    k = torch.randn(S, hkv, d, generator=g, device=DEV) * kscale
+    v = torch.randn(S, hkv, d, generator=g, device=DEV) * vscale
+    got, want = _run(q, k, v, block).double(), _dense(q, k, v)
+    # a score s = sum_d q_d k_d / sqrt(d) in fp32 has an error of about
+    # sqrt(d) 2^-24 |q_d k_d| ~ 2^-24 |s|_rms, which shifts log P; the sums of P
+    # and P.V add a few 2^-24: 16 x 2^-24 (1 + rms of the scores)
+    rel = ((got - want).norm() / want.norm()).item()
+    assert rel <= 16 * 2.0 ** -24 * (1 + kscale), rel
+
+
+@pytest.mark.parametrize("value", [2.0 ** 56, 1e30, 3.4028234e38, math.inf, -math.inf])
+def test_a_key_of_score_minus_infinity_or_far_below_drops_out(value):
+    # keys whose score is hugely negative (or -inf) get P = 0: the rows equal
+    # those computed without them, with no NaN from the parts
+    S, d = 300, 64
+    g = torch.Generator(device=DEV).manual_seed(1)
+    q = torch.rand(S, 2, d, generator=g, device=DEV) + 0.5
+    k = torch.randn(S, 1, d, generator=g, device=DEV)
+    v = torch.randn(S, 1, d, generator=g, device=DEV)
+    at = torch.tensor([7, 150, 290], device=DEV)
+    k[at] = -abs(value)
+    got = _run(q, k, v)
+    kk = k.clone()
+    kk[at] = -1e3
+    want = _run(q, kk, v)
+    assert not got.isnan().any()
+    # the scalar products add in another order (see the bound above; 4: the rms
+    # of these scores)
+    assert ((got - want).norm() / want.norm()).item() <= 32 * 2.0 ** -24 * 4
+
+
+def test_large_and_infinite_values():
+    S, d = 300, 64
+    g = torch.Generator(device=DEV).manual_seed(2)
+    q = torch.randn(S, 1, d, generator=g, device=DEV)
+    k = torch.randn(S, 1, d, generator=g, device=DEV)
+    v = torch.randn(S, 1, d, generator=g, device=DEV)
+    v[3, 0, 5] = 1e35  # finite: the result is finite
+    got, want = _run(q, k, v).double(), _dense(q, k, v)
+    assert ((got - want)[:, 0, 5].norm() / want[:, 0, 5].norm()).item() <= 64 * 2.0 ** -24
+    # every row from 3 on holds inf in that dim (rows 0 .. 2 multiply it by the
+    # P = 0 of a masked key, which is NaN, as the reference's masked tile does);
+    # the other dims stay finite
+    v[3, 0, 5] = math.inf
+    got = _run(q, k, v)
+    assert got[3:, 0, 5].isinf().all()
+    assert got[:, 0, :5].isfinite().all() and got[:, 0, 6:].isfinite().all()
+    v[3, 0, 5] = math.nan
+    got = _run(q, k, v)
+    assert got[3:, 0, 5].isnan().all() and got[:, 0, 6:].isfinite().all()
+
+
+def test_sparse_lists_in_chunks_match_one_slot_per_row():
+    # 4000 tokens of 2 heads (several chunk slots) against the same rows in a
+    # batch of enough heads for one slot per row
+    from flashprefill_amd import synth
+    spec = synth.SynthSpec(seq_lens=(4000,), num_q_heads=2, num_kv_heads=1, head_dim=64,
+                           dtype=torch.float32, seed=5)
+    q, k, v, _ = synth.make_inputs(spec, "cpu")
+    one = [t.to(DEV).unsqueeze(0) for t in (q, k, v)]
+    many = [t.repeat(16, 1, 1, 1) for t in one]
+    o1, o16 = torch.empty_like(one[0]), torch.empty_like(many[0])
+    flash_prefill(*one, o1, 128, 2, 4, 0.3, 2, 0)
+    flash_prefill(*many, o16, 128, 2, 4, 0.3, 2, 0)
+    # the same products; the chunks' merge adds a rounding per chunk
+    assert ((o1 - o16[:1]).norm() / o1.norm()).item() <= 8 * 2.0 ** -24
+    assert torch.equal(o16[0], o16[15])
