@@ -329,11 +329,10 @@ int run_pool(const fp_problem* p, const fp_ws_layout& L, void* ws, hipStream_t s
 }
 
 // The plan and the pooling of a whole-operator call: one launch (k_plan_pool)
-// for 16-bit inputs and at most kSmallPlanBatch sequences, where the plan's
-// own launch and latency are a visible part of a short call; otherwise k_plan
-// then k_pool.
+// for at most kSmallPlanBatch sequences, where the plan's own launch and
+// latency are a visible part of a short call; otherwise k_plan then k_pool.
 int run_plan_and_pool(const fp_problem* p, const fp_ws_layout& L, void* ws, hipStream_t s) {
-  if (p->dtype != FP_DTYPE_F32 && p->batch <= fp::kSmallPlanBatch) {
+  if (p->batch <= fp::kSmallPlanBatch) {
     const hipError_t e = fp::launch_plan_pool(plan_args(p, L, ws), pool_args(p, L, ws), p->dtype,
                                               p->head_dim, s);
     return e == hipSuccess ? FP_OK : hip_fail(e, "plan + pool launch");

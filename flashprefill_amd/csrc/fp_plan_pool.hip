@@ -228,8 +228,42 @@ __global__ __launch_bounds__(1024) void k_plan(PlanArgs a) {
   if (t == 0) *tab.status = s_status;
 }
 
+// A 16-byte chunk of K as E values, and the means converted back.
+template <typename T>
+struct PoolChunk {
+  static constexpr int E = 8;
+  static __device__ __forceinline__ void add(uint4 v, double (&acc)[E]) {
+    const uint16_t* e = reinterpret_cast<const uint16_t*>(&v);
+#pragma unroll
+    for (int q = 0; q < E; ++q) acc[q] += static_cast<double>(T::to_f32(e[q]));
+  }
+  static __device__ __forceinline__ uint4 mean(const double (&acc)[E], double n) {
+    uint16_t o[E];
+#pragma unroll
+    for (int q = 0; q < E; ++q) o[q] = T::from_f32(static_cast<float>(acc[q] / n));
+    return *reinterpret_cast<const uint4*>(o);
+  }
+};
+struct F32 {};
+template <>
+struct PoolChunk<F32> {
+  static constexpr int E = 4;
+  static __device__ __forceinline__ void add(uint4 v, double (&acc)[E]) {
+    acc[0] += static_cast<double>(__uint_as_float(v.x));
+    acc[1] += static_cast<double>(__uint_as_float(v.y));
+    acc[2] += static_cast<double>(__uint_as_float(v.z));
+    acc[3] += static_cast<double>(__uint_as_float(v.w));
+  }
+  static __device__ __forceinline__ uint4 mean(const double (&acc)[E], double n) {
+    return make_uint4(__float_as_uint(static_cast<float>(acc[0] / n)),
+                      __float_as_uint(static_cast<float>(acc[1] / n)),
+                      __float_as_uint(static_cast<float>(acc[2] / n)),
+                      __float_as_uint(static_cast<float>(acc[3] / n)));
+  }
+};
+
 // Mean of key block g of kv head hh (rows t0 .. t0 + rows - 1 of K), by one
-// workgroup of 256 threads = R row groups x D / 8 chunks of 16 bytes; each
+// workgroup of 256 threads = R row groups x C chunks of 16 bytes; each
 // thread sums its rows of one chunk in fp64. The R partial sums are added
 // within each wave by lane exchanges (its 64 / C row groups), then the four
 // waves' sums through LDS, and the mean sum / rows is divided in fp64 and
@@ -237,30 +271,34 @@ __global__ __launch_bounds__(1024) void k_plan(PlanArgs a) {
 // float64 -> bfloat16 / float16 cast). A 16-bit value has an 8- or 11-bit
 // significand, so a sum of at most 256 of them is exact in fp64 unless their
 // exponents span more than ~38 binades: the mean is then the correctly
-// rounded block mean whatever the order of the additions. The means are
+// rounded block mean whatever the order of the additions. fp32 keys: the fp64
+// sum is rounded once to fp32. (One thread per dim with its rows in a serial
+// chain, as fp32 keys were pooled before, took 15-32 us for 4K tokens x 2 KV
+// heads; this way 4 us, beside the plan in one launch.) The means are
 // stored chunk-major (16-byte chunk c of key block g and kv head hh at entry
 // g of chunk row hh * C + c), so that the search kernel's loads of 32
 // consecutive keys' chunk are contiguous.
 template <typename T, int D>
 __device__ __forceinline__ void pool_block(const PoolArgs& a, int64_t g, int hh, int64_t t0,
                                            int rows) {
-  constexpr int C = D / 8;    // 16-byte chunks per head row
+  typedef PoolChunk<T> PC;
+  constexpr int E = PC::E;    // values per chunk
+  constexpr int C = D / E;    // 16-byte chunks per head row
   constexpr int R = 256 / C;  // row groups
-  __shared__ double red[3][C][8];  // sums of waves 1 .. 3
+  __shared__ double red[3][C][E];  // sums of waves 1 .. 3
   const int t = threadIdx.x, c = t % C, rg = t / C;
-  const uint16_t* src = a.k + t0 * a.kst + hh * a.khs + c * 8;
-  double acc[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-  for (int r = rg; r < rows; r += R) {
-    const uint4 v = ld16(src + static_cast<int64_t>(r) * a.kst);
-    const uint16_t* e = reinterpret_cast<const uint16_t*>(&v);
+  const char* src = reinterpret_cast<const char*>(a.k) +
+                    (t0 * a.kst + hh * a.khs) * (16 / E) + c * 16;
+  const int64_t row = a.kst * (16 / E);  // bytes between rows
+  double acc[E];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) acc[q] += static_cast<double>(T::to_f32(e[q]));
-  }
+  for (int q = 0; q < E; ++q) acc[q] = 0.0;
+  for (int r = rg; r < rows; r += R) PC::add(ld16(src + static_cast<int64_t>(r) * row), acc);
   // lanes c, c + C, ... of a wave hold the same chunk: xor exchanges over the
   // lane bits above log2(C) add the wave's row groups
   const int w = t >> 6;
 #pragma unroll
-  for (int q = 0; q < 8; ++q) {
+  for (int q = 0; q < E; ++q) {
     if constexpr (C <= 16) acc[q] += xchg_xor_d<16>(acc[q]);
     if constexpr (C <= 8) acc[q] += xchg_xor_d<8>(acc[q]);
     const uint64_t u = __double_as_longlong(acc[q]);
@@ -269,19 +307,15 @@ __device__ __forceinline__ void pool_block(const PoolArgs& a, int64_t g, int hh,
   }
   if (w > 0 && (t & 63) < C) {
 #pragma unroll
-    for (int q = 0; q < 8; ++q) red[w - 1][c][q] = acc[q];
+    for (int q = 0; q < E; ++q) red[w - 1][c][q] = acc[q];
   }
   __syncthreads();
   if (t < C) {
-    const double n = static_cast<double>(rows);
 #pragma unroll
-    for (int q = 0; q < 8; ++q) acc[q] += red[0][c][q] + red[1][c][q] + red[2][c][q];
-    uint16_t o[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) o[q] = T::from_f32(static_cast<float>(acc[q] / n));
+    for (int q = 0; q < E; ++q) acc[q] += red[0][c][q] + red[1][c][q] + red[2][c][q];
     // chunk-major: chunk c of (g, hh) is entry g of chunk row hh * C + c
-    uint16_t* out = a.mk + ((hh * C + c) * a.nb_sum_cap + g) * 8;
-    st16(out, *reinterpret_cast<const uint4*>(o));
+    st16(reinterpret_cast<char*>(a.mk) + ((hh * C + c) * a.nb_sum_cap + g) * 16,
+         PC::mean(acc, static_cast<double>(rows)));
   }
 }
 
@@ -493,31 +527,6 @@ __global__ __launch_bounds__(256) void k_plan_pool(PlanArgs pa, PoolArgs a) {
                    min(a.block * a.ratio, sp.len[b] - i * a.block));
 }
 
-// fp32 keys: the block mean summed in fp64 (in row order) and rounded once to
-// fp32, one thread per dim of one (key block, kv head) per workgroup.
-__global__ __launch_bounds__(256) void k_pool_f32(PoolArgs a, int head_dim) {
-  const int64_t g = blockIdx.x / a.Hkv;
-  const int hh = static_cast<int>(blockIdx.x % a.Hkv);
-  const int64_t nsum = a.tab.seq_tile[a.B];
-  if (g >= nsum) return;
-  const int b = find_seq(a.tab.seq_tile, a.B, g);
-  const int i = static_cast<int>(g - a.tab.seq_tile[b]);
-  if (i % a.ratio) return;
-  const int L = a.tab.seq_len[b];
-  const int64_t t0 = a.tab.seq_start[b] + static_cast<int64_t>(i) * a.block;
-  const int rows = min(a.block * a.ratio, L - i * a.block);
-  const float* k = reinterpret_cast<const float*>(a.k);
-  // chunk-major: dims 4c .. 4c+3 of (g, hh) are entry g of chunk row hh * d / 4 + c
-  float* out = reinterpret_cast<float*>(a.mk);
-  for (int x = threadIdx.x; x < head_dim; x += blockDim.x) {
-    const float* src = k + t0 * a.kst + hh * a.khs + x;
-    double sum = 0.0;
-    for (int r = 0; r < rows; ++r) sum += static_cast<double>(src[static_cast<int64_t>(r) * a.kst]);
-    const int64_t row = static_cast<int64_t>(hh) * (head_dim / 4) + x / 4;
-    out[(row * a.nb_sum_cap + g) * 4 + x % 4] = static_cast<float>(sum / static_cast<double>(rows));
-  }
-}
-
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
@@ -534,6 +543,11 @@ hipError_t launch_plan_pool(const PlanArgs& pa, const PoolArgs& a, int dtype, in
                             hipStream_t s) {
   // one workgroup per (key block, kv head) of the capacity, plus the table writer
   const dim3 g(static_cast<unsigned>(a.nb_sum_cap * a.Hkv + 1)), blk(256);
+  if (dtype == FP_DTYPE_F32) {  // head_dim 64 or 128
+    if (head_dim == 128) hipLaunchKernelGGL((k_plan_pool<F32, 128>), g, blk, 0, s, pa, a);
+    else hipLaunchKernelGGL((k_plan_pool<F32, 64>), g, blk, 0, s, pa, a);
+    return hipGetLastError();
+  }
   with_head_dim(head_dim, [&](auto dc) {
     constexpr int D = decltype(dc)::value;
     if (dtype == FP_DTYPE_BF16) hipLaunchKernelGGL((k_plan_pool<BF16, D>), g, blk, 0, s, pa, a);
@@ -548,7 +562,8 @@ hipError_t launch_pool(const PoolArgs& a, int dtype, int head_dim, int64_t grid,
   // one workgroup per (key block, kv head)
   const dim3 g(static_cast<unsigned>(grid * a.Hkv)), blk(256);
   if (dtype == FP_DTYPE_F32) {
-    hipLaunchKernelGGL(k_pool_f32, g, blk, 0, s, a, head_dim);
+    if (head_dim == 128) hipLaunchKernelGGL((k_pool<F32, 128>), g, blk, 0, s, a);
+    else hipLaunchKernelGGL((k_pool<F32, 64>), g, blk, 0, s, a);
   } else {
     with_head_dim(head_dim, [&](auto dc) {
       constexpr int D = decltype(dc)::value;
