@@ -240,7 +240,13 @@ struct PoolChunk {
   static __device__ __forceinline__ uint4 mean(const double (&acc)[E], double n) {
     uint16_t o[E];
 #pragma unroll
-    for (int q = 0; q < E; ++q) o[q] = T::from_f32(static_cast<float>(acc[q] / n));
+    for (int q = 0; q < E; ++q) {
+      float m = static_cast<float>(acc[q] / n);
+      // both roundings, fp64 -> fp32 -> T: kept apart from the next conversion,
+      // which the compiler otherwise merges into one fp64 -> bf16 rounding
+      asm volatile("" : "+v"(m));
+      o[q] = T::from_f32(m);
+    }
     return *reinterpret_cast<const uint4*>(o);
   }
 };
