@@ -25,7 +25,9 @@ LIB_PATH = PKG_DIR / LIB_NAME
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 BUILD_DIR = PKG_DIR / "_build"
-FILE_FLAGS: dict = {}
+# head dim 256: more than 256 registers per wave, where the compiler otherwise
+# gives every MFMA an accumulation-register result
+FILE_FLAGS: dict = {"fp_attn_d256.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 
 def sources():

@@ -189,6 +189,10 @@ hipError_t launch_attn(const AttnArgs& a, int dtype, int head_dim, int block, in
                        bool persist, hipStream_t s);
 // combines the chunk partials of the split rows into their output rows
 hipError_t launch_merge(const AttnArgs& a, int dtype, int head_dim, int block, hipStream_t s);
+// head dim 256 (fp_attn_d256.hip)
+hipError_t launch_attn_d256(const AttnArgs& a, int dtype, int block, int64_t grid, bool persist,
+                            hipStream_t s);
+hipError_t launch_merge_d256(const AttnArgs& a, int dtype, int block, hipStream_t s);
 hipError_t launch_attn_f32(const AttnArgs& a, int head_dim, int block, hipStream_t s);
 
 }  // namespace fp
