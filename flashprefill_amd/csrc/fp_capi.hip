@@ -528,22 +528,34 @@ int paged_valid(const fp_paged_args* a) {
   return FP_OK;
 }
 
-// Row tiles and chunk slots of a paged call. Tiles: 16 rows (query tokens x
-// the query heads of a KV head) of one sequence; at most T G / 16 + B of them,
-// and no more than each token's rows on their own would make. Chunk slots:
+// Row tiles and chunk slots of a paged call. Tiles: `rt` rows (query tokens x
+// the query heads of a KV head) of one sequence; at most T G / rt + B of them,
+// and no more than each token's rows on their own would make. rt is 16
+// (k_paged, decode) or, from kManyRows rows per sequence on average and up to
+// head_dim 128 (O^T of 256 dims and three parts of P do not fit a wave's 256
+// registers), 128 (k_paged_rows). Chunk slots:
 // about kTarget workgroups in all (several rounds of the card's ~768 resident
 // ones, so that sequences of different lengths balance), no more than
-// kPagedMaxChunks, and none shorter than kPagedMinChunk keys.
+// kPagedMaxChunks, and none shorter than kPagedMinChunk keys. (k_paged_rows:
+// its 512 resident workgroups; every chunk costs a pass over fp32 partials of all
+// its rows: one sequence of 8,192 tokens with 512 new ones, 32 q / 8 kv heads, 160
+// us with 512, 176 with 1024, 205 with 2048.) The line between the kernels: 8
+// sequences of 3,000 tokens, 32 q / 8 kv heads, with 4, 8, 16 and 64 queries each
+// (16, 32, 64 and 256 rows): k_paged 147 (32 of 4,000), 49, 84 and 254 us,
+// k_paged_rows 153, 46, 45 and 90.
 struct PagedSplit {
+  bool many;  // k_paged_rows
   int64_t tiles;
   int nc;
   size_t bytes;
 };
 PagedSplit paged_split(const fp_paged_args* a) {
-  constexpr int64_t kTarget = 8192;
+  constexpr int64_t kManyRows = 32;
   PagedSplit r;
   const int64_t G = a->num_q_heads / a->num_kv_heads, T = a->num_tokens;
-  r.tiles = std::min<int64_t>(T * ((G + 15) / 16), T * G / 16 + a->batch);
+  r.many = a->head_dim <= 128 && T * G >= kManyRows * a->batch;
+  const int64_t kTarget = r.many ? 512 : 8192, rt = r.many ? 128 : 16;
+  r.tiles = std::min<int64_t>(T * ((G + rt - 1) / rt), T * G / rt + a->batch);
   const int64_t longest = static_cast<int64_t>(a->table_width) * a->block_size;
   const int64_t wgs = std::max<int64_t>(1, r.tiles * a->num_kv_heads);
   int64_t nc = std::min<int64_t>(fp::kPagedMaxChunks, (kTarget + wgs - 1) / wgs);
@@ -728,8 +740,8 @@ int fp_paged_attention(const fp_paged_args* a, void* ws, void* stream) {
   r.part = static_cast<float*>(ws);
   r.ml = sp.nc > 1 ? static_cast<float*>(ws) + a->num_tokens * a->num_q_heads * sp.nc * a->head_dim
                    : nullptr;
-  const hipError_t e = fp::launch_paged(r, a->dtype, a->head_dim, sp.tiles,
-                                        static_cast<hipStream_t>(stream));
+  const auto launch = sp.many ? fp::launch_paged_rows : fp::launch_paged;
+  const hipError_t e = launch(r, a->dtype, a->head_dim, sp.tiles, static_cast<hipStream_t>(stream));
   return e == hipSuccess ? FP_OK : hip_fail(e, "paged attention launch");
 }
 

@@ -177,6 +177,8 @@ auto with_head_dim(int head_dim, F&& f) {
 
 hipError_t launch_plan(const PlanArgs& a, hipStream_t s);
 hipError_t launch_rope(const RopeArgs& a, int dtype, hipStream_t s);
+hipError_t launch_paged_rows(const PagedArgs& a, int dtype, int head_dim, int64_t tiles,
+                             hipStream_t s);
 hipError_t launch_paged(const PagedArgs& a, int dtype, int head_dim, int64_t tiles, hipStream_t s);
 hipError_t launch_kv_cache_write(const KvCacheArgs& a, hipStream_t s);
 hipError_t launch_pool(const PoolArgs& a, int dtype, int head_dim, int64_t grid, hipStream_t s);

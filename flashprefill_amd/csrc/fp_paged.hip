@@ -482,6 +482,316 @@ __global__ __launch_bounds__(256) void k_paged_merge(PagedArgs a) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// Many query rows per sequence (prefix-cached prefill)
+// ---------------------------------------------------------------------------
+// P as three parts of the input type that add up to it: fp32 has 24 significand
+// bits, bf16 parts hold 8 each, fp16 parts 11 each. fp16 lacks fp32's exponents,
+// so P enters scaled by 2^14 (kPShift; P <= 2^14 < 65504, and a part below
+// fp16's last step, 2^-24, is 2^-38 of the row's largest P).
+template <typename T>
+struct PParts;
+template <>
+struct PParts<BF16> {
+  static constexpr float kPShift = 0.0f;
+};
+template <>
+struct PParts<F16> {
+  static constexpr float kPShift = 14.0f;
+};
+template <typename T>
+__device__ __forceinline__ void part_pair(float x0, float x1, uint32_t (&u)[3]) {
+#pragma unroll
+  for (int p = 0; p < 3; ++p) {
+    u[p] = pack2<T>(x0, x1);
+    x0 -= T::to_f32(static_cast<uint16_t>(u[p]));
+    x1 -= T::to_f32(static_cast<uint16_t>(u[p] >> 16));
+  }
+}
+
+// One workgroup (4 waves) per (128-row tile of the G query heads of a KV head,
+// KV head, chunk of keys), in the orientation of k_attn: wave w owns rows
+// 32 w .. 32 w + 31, S^T = K . Q^T and O^T += V^T . P^T on 32x32x16 MFMA, K and V
+// in 64-key tiles through LDS (direct-to-LDS loads, two buffers: a tile lands
+// while the one before it is used; one barrier per tile). The rows of a tile
+// share every K / V byte, where k_paged reads them once per 16 rows. P stays
+// fp32: P.V runs on its three exact 16-bit parts (48 of the 64 MFMAs of a tile
+// and wave at d = 128). Bound by these MFMAs and the instructions that form the
+// parts. Measured (one MI355X): 500 new tokens each on 6,144, 2,500 and 1,111
+// cached ones (28 q / 4 kv heads, d = 128) 504 us with k_paged, 182 here; 4 x
+// 2,048 new of 4,096 (32 q / 8 kv) 3,045 -> 890 us = 463 TFLOP/s (924 of MFMAs).
+template <typename T, int D, bool P16>
+__global__ __launch_bounds__(256, 2) void k_paged_rows(PagedArgs a) {
+  constexpr int KT = 64, TT = KT / 32;
+  constexpr int KS = D / 16, DT = D / 32, CH = D / 8;
+  constexpr int RPW = 64 / CH;             // rows per load instruction
+  constexpr int NI = KT * CH / 64 / 4;     // load instructions per wave and tile
+  static_assert(NI * RPW == 16, "a wave loads 16 consecutive keys of a tile");
+  __shared__ uint4 sk[2][KT * CH];
+  __shared__ uint4 sv[2][KT * CH];
+  const int h = static_cast<int>(blockIdx.x % a.Hkv);
+  const int64_t x = blockIdx.x / a.Hkv;
+  const int c = static_cast<int>(blockIdx.y);
+  const PagedTile tile = paged_find(a, 128, x, -1);
+  if (tile.b < 0) return;
+  const PagedSeq& sq = tile.s;
+  const int nk = static_cast<int>(sq.nk), nq = sq.nq;
+  const int k0 = c * tile.chunk;
+  if (k0 >= nk && c > 0) return;
+  const bool single = nk <= tile.chunk;
+  const int t = threadIdx.x, lane = t & 63;
+  const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int half = lane >> 5, l32 = lane & 31;
+  const int rows = nq * a.G;
+
+  // this lane's query row and its last visible key
+  const int rr = tile.tl * 128 + 32 * w + l32;
+  const bool rvalid = rr < rows;
+  const int qi = (rvalid ? rr : rows - 1) / a.G;
+  const int64_t tok = sq.q0 + qi;
+  const int hq = h * a.G + (rvalid ? rr : rows - 1) % a.G;
+  const int lim = nk - nq + qi;
+  // the wave's first and last visible keys' bounds (wave-uniform)
+  const int r0 = min(tile.tl * 128 + 32 * w, rows - 1), r1 = min(tile.tl * 128 + 32 * w + 31, rows - 1);
+  const int lim_lo = __builtin_amdgcn_readfirstlane(nk - nq + r0 / a.G);
+  const int lim_hi = __builtin_amdgcn_readfirstlane(nk - nq + r1 / a.G);
+  // keys past the last row of the tile are visible to none of its rows
+  const int last_row = min(tile.tl * 128 + 127, rows - 1);
+  const int k1 = __builtin_amdgcn_readfirstlane(
+      min(min(k0 + tile.chunk, nk), max(nk - nq + last_row / a.G + 1, 0)));
+
+  typename T::vec8 qb[KS];
+  {
+    const uint16_t* qp = static_cast<const uint16_t*>(a.q) + tok * a.qst +
+                         static_cast<int64_t>(hq) * a.qhs + 8 * half;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) qb[s] = as_vec8<T>(rvalid ? ld16(qp + 16 * s) : zero4());
+  }
+  f32x16 o[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) o[dt] = f32x16{};
+  float m_run = -INFINITY, l_part = 0.0f;
+  bool bad = false;
+
+  const int64_t row = static_cast<int64_t>(tile.b) * a.table_stride;
+  const uint16_t* kc = static_cast<const uint16_t*>(a.kc) + static_cast<int64_t>(h) * a.kch;
+  const uint16_t* vc = static_cast<const uint16_t*>(a.vc) + static_cast<int64_t>(h) * a.vch;
+  // the lane's byte offsets in the wave's 16 keys (P16)
+  uint32_t koff[NI], voff[NI];
+#pragma unroll
+  for (int q = 0; q < NI; ++q) {
+    const int r = q * RPW + lane / CH;
+    const int ch = 8 * ((lane % CH) ^ swz<D>(16 * w + r));
+    koff[q] = 2 * (static_cast<uint32_t>(r) * static_cast<uint32_t>(a.kcs) + ch);
+    voff[q] = 2 * (static_cast<uint32_t>(r) * static_cast<uint32_t>(a.vcs) + ch);
+  }
+  const int last16 = (nk - 1) & ~15;
+  // tile of keys base .. base + 63 into buffer `buf`; keys past the sequence
+  // read its last 16-key group (P16: slots past the end are masked and their V
+  // zeroed below) or its last key
+  auto issue = [&](int base, int buf) {
+    if constexpr (P16) {
+      const int tb = min(base + 16 * w, last16);
+      const int64_t pg = paged_page<true>(a, row, tb, bad);
+      const int in = a.bs_shift >= 0 ? tb & (a.bs - 1) : tb % a.bs;
+      uint64_t kb = scalar_addr(kc + pg * a.kcb + static_cast<int64_t>(in) * a.kcs);
+      uint64_t vb = scalar_addr(vc + pg * a.vcb + static_cast<int64_t>(in) * a.vcs);
+      const uint32_t kl = lds_addr(sk[buf] + w * NI * 64), vl = lds_addr(sv[buf] + w * NI * 64);
+      // five wait states between the readfirstlane of the bases and their use
+      asm volatile("s_nop 4" : "+s"(kb), "+s"(vb));
+#pragma unroll
+      for (int q = 0; q < NI; ++q) dma16_sbase_m0(kl + q * 1024, kb, koff[q]);
+#pragma unroll
+      for (int q = 0; q < NI; ++q) dma16_sbase_m0(vl + q * 1024, vb, voff[q]);
+    } else {
+#pragma unroll
+      for (int q = 0; q < NI; ++q) {
+        const int r = 16 * w + q * RPW + lane / CH;
+        const int key = min(base + r, nk - 1);
+        const int64_t pg = paged_page<false>(a, row, key, bad);
+        const int in = key % a.bs, ch = 8 * ((lane % CH) ^ swz<D>(r));
+        dma16_vaddr(sk[buf] + (w * NI + q) * 64, kc + pg * a.kcb + static_cast<int64_t>(in) * a.kcs + ch);
+        dma16_vaddr(sv[buf] + (w * NI + q) * 64, vc + pg * a.vcb + static_cast<int64_t>(in) * a.vcs + ch);
+      }
+    }
+  };
+  const int g16 = lane >> 4, i16 = lane & 15;
+  const int tr_row = 4 * (g16 >> 1) + (i16 >> 2);
+  const int tr_col = 16 * (g16 & 1) + 4 * (i16 & 3);
+
+  if (k0 < k1) issue(k0, 0);
+  int buf = 0;
+  for (int base = k0; base < k1; base += KT, buf ^= 1) {
+    // this tile has landed for every wave, and every wave is done with the other
+    // buffer
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (base + KT < k1) issue(base + KT, buf ^ 1);
+    if (base + KT > nk) {  // V of slots past the sequence: 0 (they may hold anything)
+      for (int i = t; i < KT * CH; i += 256)
+        if (base + i / CH >= nk) sv[buf][i] = zero4();
+      lds_barrier();
+    }
+    if (base > lim_hi) continue;  // no key of this tile is visible to the wave
+    f32x16 s[TT];
+#pragma unroll
+    for (int t4 = 0; t4 < TT; ++t4) s[t4] = f32x16{};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int t4 = 0; t4 < TT; ++t4) {
+        const int r = 32 * t4 + l32;
+        const uint4 kop = sk[buf][r * CH + ((2 * ks + half) ^ swz<D>(r))];
+        s[t4] = T::mfma32(as_vec8<T>(kop), qb[ks], s[t4]);
+      }
+    float mx = -INFINITY;
+    if (base + KT - 1 > lim_lo) {
+#pragma unroll
+      for (int t4 = 0; t4 < TT; ++t4)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int key = base + 32 * t4 + 8 * (v >> 2) + 4 * half + (v & 3);
+          s[t4][v] = key > lim ? -INFINITY : s[t4][v] * a.scale_log2;
+          mx = fmaxf(mx, s[t4][v]);
+        }
+    } else {
+#pragma unroll
+      for (int t4 = 0; t4 < TT; ++t4)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          s[t4][v] *= a.scale_log2;
+          mx = fmaxf(mx, s[t4][v]);
+        }
+    }
+    const float m_new = fmaxf(m_run, pair32_max(mx));
+    if (__ballot(m_new > m_run) != 0) {
+      const float ms = m_new == -INFINITY ? 0.0f : m_new;
+      const float alpha = __builtin_amdgcn_exp2f(m_run - ms);
+      m_run = m_new;
+      l_part *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[dt][v] *= alpha;
+    }
+    // rows with no visible key yet keep m = -inf: their P is 0
+    const float ms = (m_run == -INFINITY ? 0.0f : m_run) - PParts<T>::kPShift;
+#pragma unroll
+    for (int t4 = 0; t4 < TT; ++t4) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        s[t4][v] = __builtin_amdgcn_exp2f(s[t4][v] - ms);
+        l_part += s[t4][v];
+      }
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh) {
+        uint32_t u[4][3];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          part_pair<T>(s[t4][8 * hh + 2 * e], s[t4][8 * hh + 2 * e + 1], u[e]);
+        typename T::vec8 pb[3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p)
+          pb[p] = as_vec8<T>(make_uint4(u[0][p], u[1][p], u[2][p], u[3][p]));
+        const uint16_t* sv16 = reinterpret_cast<const uint16_t*>(sv[buf]);
+        const int r = 32 * t4 + 16 * hh + tr_row;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+          const int xx = 32 * dt + tr_col;
+          const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (__attribute__((address_space(3))) i16x4*)(sv16 + tile_elem<D>(r, xx)));
+          const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (__attribute__((address_space(3))) i16x4*)(sv16 + tile_elem<D>(r + 8, xx)));
+          const uint2 lo2 = __builtin_bit_cast(uint2, lo), hi2 = __builtin_bit_cast(uint2, hi);
+          const typename T::vec8 va = as_vec8<T>(make_uint4(lo2.x, lo2.y, hi2.x, hi2.y));
+          o[dt] = T::mfma32(va, pb[2], o[dt]);
+          o[dt] = T::mfma32(va, pb[1], o[dt]);
+          o[dt] = T::mfma32(va, pb[0], o[dt]);
+        }
+      }
+    }
+  }
+
+  float l = pair32_sum(l_part);
+  if (__ballot(bad) != 0) l = __uint_as_float(0x7fc00000u);
+  if (!rvalid) return;
+  if (single) {
+    const float rcp = 1.0f / l;
+    uint16_t* op = static_cast<uint16_t*>(a.o) + tok * a.ost + static_cast<int64_t>(hq) * a.ohs;
+    const float nan = __uint_as_float(0x7fc00000u);
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int g4 = 0; g4 < 4; ++g4) {
+        float y[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          y[e] = o[dt][4 * g4 + e] * rcp;
+          if (nk == 0) y[e] = sq.bad ? nan : 0.0f;
+        }
+        *reinterpret_cast<uint2*>(op + 32 * dt + 8 * g4 + 4 * half) =
+            make_uint2(pack2<T>(y[0], y[1]), pack2<T>(y[2], y[3]));
+      }
+  } else {
+    const int64_t slot = (tok * a.Hq + hq) * a.nc + c;
+    float* pp = a.part + slot * D;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int g4 = 0; g4 < 4; ++g4)
+        *reinterpret_cast<float4*>(pp + 32 * dt + 8 * g4 + 4 * half) =
+            make_float4(o[dt][4 * g4], o[dt][4 * g4 + 1], o[dt][4 * g4 + 2], o[dt][4 * g4 + 3]);
+    if (half == 0) {
+      a.ml[2 * slot] = m_run;
+      a.ml[2 * slot + 1] = l;
+    }
+  }
+}
+
+// Output rows of k_paged_rows: one wave per row (four per workgroup), its
+// chunks (few) in turn; the arithmetic of k_paged_merge.
+template <typename T, int D>
+__global__ __launch_bounds__(256) void k_paged_merge_rows(PagedArgs a) {
+  constexpr int XD = D / 64;  // dims per lane
+  const int64_t r = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  if (r >= a.T * a.Hq) return;
+  const int64_t tok = r / a.Hq;
+  const int hq = static_cast<int>(r % a.Hq), lane = threadIdx.x & 63;
+  const PagedTile tile = paged_find(a, 128, 0, tok);
+  if (tile.b < 0) return;
+  const int nk = static_cast<int>(tile.s.nk);
+  if (nk <= tile.chunk) return;
+  const int n = min((nk + tile.chunk - 1) / tile.chunk, a.nc);
+  const int64_t slot = r * a.nc;
+  float M = -INFINITY;
+  for (int c = 0; c < n; ++c) M = fmaxf(M, a.ml[2 * (slot + c)]);
+  float L = 0.0f, acc[XD];
+#pragma unroll
+  for (int q = 0; q < XD; ++q) acc[q] = 0.0f;
+#pragma unroll 4
+  for (int c = 0; c < n; ++c) {
+    const float m = a.ml[2 * (slot + c)], l = a.ml[2 * (slot + c) + 1];
+    const float f = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - M);
+    L += m == -INFINITY ? l : f * l;
+#pragma unroll
+    for (int q = 0; q < XD; ++q) acc[q] += f * a.part[(slot + c) * D + XD * lane + q];
+  }
+  uint16_t* op = static_cast<uint16_t*>(a.o) + tok * a.ost + static_cast<int64_t>(hq) * a.ohs + XD * lane;
+  const float rcp = 1.0f / L;
+  if constexpr (XD == 2) *reinterpret_cast<uint32_t*>(op) = pack2<T>(acc[0] * rcp, acc[1] * rcp);
+  else op[0] = T::from_f32(acc[0] * rcp);
+}
+
+template <typename T, int D>
+hipError_t launch_paged_rows_t(const PagedArgs& a, int64_t tiles, hipStream_t s) {
+  const dim3 grid(static_cast<unsigned>(tiles * a.Hkv), static_cast<unsigned>(a.nc));
+  if (a.bs % 16 == 0) hipLaunchKernelGGL((k_paged_rows<T, D, true>), grid, dim3(256), 0, s, a);
+  else hipLaunchKernelGGL((k_paged_rows<T, D, false>), grid, dim3(256), 0, s, a);
+  if (a.nc > 1)
+    hipLaunchKernelGGL((k_paged_merge_rows<T, D>),
+                       dim3(static_cast<unsigned>((a.T * a.Hq + 3) / 4)), dim3(256), 0, s, a);
+  return hipGetLastError();
+}
+
 template <typename T, int D>
 hipError_t launch_paged_t(const PagedArgs& a, int64_t tiles, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>(tiles * a.Hkv), static_cast<unsigned>(a.nc));
@@ -491,6 +801,15 @@ hipError_t launch_paged_t(const PagedArgs& a, int64_t tiles, hipStream_t s) {
     hipLaunchKernelGGL((k_paged_merge<T, D>), dim3(static_cast<unsigned>(a.T * a.Hq)), dim3(256), 0,
                        s, a);
   return hipGetLastError();
+}
+
+hipError_t launch_paged_rows(const PagedArgs& a, int dtype, int head_dim, int64_t tiles,
+                             hipStream_t s) {
+  if (head_dim == 128)
+    return dtype == FP_DTYPE_BF16 ? launch_paged_rows_t<BF16, 128>(a, tiles, s)
+                                  : launch_paged_rows_t<F16, 128>(a, tiles, s);
+  return dtype == FP_DTYPE_BF16 ? launch_paged_rows_t<BF16, 64>(a, tiles, s)
+                                : launch_paged_rows_t<F16, 64>(a, tiles, s);
 }
 
 hipError_t launch_paged(const PagedArgs& a, int dtype, int head_dim, int64_t tiles, hipStream_t s) {

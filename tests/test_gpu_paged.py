@@ -103,6 +103,29 @@ def test_several_queries(lens, news, hq, hkv, d, dtype):
     _check(_case(lens, news, hq, hkv, d, 16, dtype), 1 / math.sqrt(d))
 
 
+@pytest.mark.parametrize("page", [1, 16, 24, 64])
+@pytest.mark.parametrize("d,dtype", [(128, torch.bfloat16), (64, torch.float16), (128, torch.float16),
+                                     (64, torch.bfloat16)])
+def test_many_rows_at_tile_edges(page, d, dtype):
+    # 128-row tiles (31, 32, 33, 64 queries x 4 heads), 64-key tiles (sequence
+    # ends one before, at and after a boundary, inside a page), one chunk and
+    # several; queries that see no key (nk < nq)
+    for lens, news in (([127, 128, 129, 64], [31, 32, 33, 64]), ([1000, 65, 320], [65, 65, 1]),
+                       ([2049, 30], [97, 40])):
+        _check(_case(lens, news, 8, 2, d, page, dtype, seed=page), 1 / math.sqrt(d))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("news", [1, 40])
+@pytest.mark.parametrize("scale", [0.5, -0.3, 1e-3])
+def test_peaked_and_flat_rows(dtype, news, scale):
+    # sharp softmax rows (most P far below the largest), a negative scale and
+    # nearly uniform rows; V of one sign, so that small P add up
+    q, kc, vc, cu, used, table = _case([3000, 700], [news, news], 8, 2, 128, 16, dtype, seed=9)
+    vc = vc.abs()
+    _check((q, kc, vc, cu, used, table), scale)
+
+
 def test_wide_table_and_many_sequences():
     # a table far wider than the sequences (a server's limit), and more
     # sequences than one round of the tile search covers
