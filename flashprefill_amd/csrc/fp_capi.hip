@@ -237,8 +237,9 @@ fp::SeqTables tables(const fp_ws_layout& L, void* ws) {
 
 // Workgroups of the attention kernel resident on the current device at once:
 // two per CU at block 128 (64 KB of LDS, 4 waves), four at block 64 (32 KB,
-// 2 waves), half that at d = 256 (one wave per SIMD, twice the LDS), rounded
-// up to a multiple of the 8 XCDs. The CU count is read once per device.
+// 2 waves), half that at d = 256 (one wave per SIMD, twice the LDS), half as
+// many again at d = 64 (three waves per SIMD, half the LDS), rounded up to a
+// multiple of the 8 XCDs. The CU count is read once per device.
 int resident_attn_workgroups(int block, int head_dim, int64_t* out) {
   constexpr int kDevs = 64;
   static std::mutex mu;
@@ -255,7 +256,8 @@ int resident_attn_workgroups(int block, int head_dim, int64_t* out) {
     if (n < 1) return fail(FP_E_LAUNCH, "device reports %d CUs", n);
     cus[dev] = n;
   }
-  const int64_t per_cu = (block == 128 ? 2 : 4) / (head_dim == 256 ? 2 : 1);
+  // waves per SIMD x 4 SIMDs / waves per workgroup
+  const int64_t per_cu = (head_dim == 256 ? 4 : head_dim == 64 ? 12 : 8) / (block / 32);
   *out = (cus[dev] * per_cu + 7) / 8 * 8;
   return FP_OK;
 }

@@ -1,0 +1,48 @@
+"""head_dim 64 attention in 64-key passes (block 128) and at three waves per SIMD
+(blocks 64 and 128): lengths around every 32- and 64-key boundary of the first
+blocks, and enough rows for the persistent grid, against float32 causal
+attention over every block (alpha 0)."""
+
+import math
+
+import pytest
+import torch
+
+from flashprefill_amd import flash_prefill_varlen_func
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("block", [64, 128])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("lens,hq,hkv", [([1, 31, 32, 33, 63, 64, 65], 4, 2),
+                                         ([96, 127, 128, 129, 191, 192, 193], 4, 1),
+                                         ([255, 256, 257, 320, 0, 385], 6, 3),
+                                         ([3000, 2900], 32, 8)])
+def test_dense_rows(lens, hq, hkv, block, dtype):
+    g = torch.Generator(device=DEV).manual_seed(sum(lens) + block)
+    T, d = sum(lens), 64
+    q = torch.randn(T, hq, d, generator=g, device=DEV).to(dtype)
+    k = torch.randn(T, hkv, d, generator=g, device=DEV).to(dtype)
+    v = torch.randn(T, hkv, d, generator=g, device=DEV).to(dtype)
+    cu = [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    o = torch.full_like(q, float("nan"))
+    flash_prefill_varlen_func(q, k, v, o, torch.tensor(cu, dtype=torch.int32, device=DEV),
+                              max(lens), 0.0, block)
+    for b, n in enumerate(lens):
+        if n == 0:
+            continue
+        sl = slice(cu[b], cu[b + 1])
+        qf, kf, vf = [t[sl].float().permute(1, 0, 2) for t in (q, k, v)]
+        kf, vf = kf.repeat_interleave(hq // hkv, 0), vf.repeat_interleave(hq // hkv, 0)
+        s = torch.matmul(qf, kf.transpose(1, 2).contiguous()) / math.sqrt(d)
+        s = s.masked_fill(torch.ones(n, n, dtype=torch.bool, device=DEV).triu(1), -math.inf)
+        err = (o[sl].float() - torch.matmul(torch.softmax(s, -1), vf).permute(1, 0, 2)).abs()
+        # P rounded to the input type against fp32 weights that sum to 1, and
+        # one rounding of the result: 2^-9 (2^-12) of |v| <= ~5 each, as a bound
+        # on every element and a tenth of it on the mean
+        bar = 2.0 ** -8 * 5 if dtype == torch.bfloat16 else 2.0 ** -11 * 5
+        assert err.max().item() <= bar and err.mean().item() <= bar / 10, (b, n, err.max())
