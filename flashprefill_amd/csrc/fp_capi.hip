@@ -330,19 +330,6 @@ int run_pool(const fp_problem* p, const fp_ws_layout& L, void* ws, hipStream_t s
   return e == hipSuccess ? FP_OK : hip_fail(e, "pool launch");
 }
 
-// The plan and the pooling of a whole-operator call: one launch (k_plan_pool)
-// for at most kSmallPlanBatch sequences, where the plan's own launch and
-// latency are a visible part of a short call; otherwise k_plan then k_pool.
-int run_plan_and_pool(const fp_problem* p, const fp_ws_layout& L, void* ws, hipStream_t s) {
-  if (p->batch <= fp::kSmallPlanBatch) {
-    const hipError_t e = fp::launch_plan_pool(plan_args(p, L, ws), pool_args(p, L, ws), p->dtype,
-                                              p->head_dim, s);
-    return e == hipSuccess ? FP_OK : hip_fail(e, "plan + pool launch");
-  }
-  const int rc = run_plan(p, L, ws, s);
-  return rc != FP_OK ? rc : run_pool(p, L, ws, s);
-}
-
 fp::SearchArgs search_args(const fp_problem* p, const fp_ws_layout& L, void* ws) {
   fp::SearchArgs a;
   memset(&a, 0, sizeof(a));
@@ -383,6 +370,40 @@ int run_search(const fp_problem* p, const fp_ws_layout& L, void* ws, float* dp, 
                                          static_cast<int64_t>(p->num_q_heads) * L.nb_sum_cap,
                                          from_scores, s);
   return e == hipSuccess ? FP_OK : hip_fail(e, "search launch");
+}
+
+// Whether the rules alone keep every block of every row, whatever the scores:
+// every row is one of its sequence's last_n rows or has no block between the
+// sink and the window, in sequences of up to nb_max blocks (2 + 4 + 2 blocks,
+// i.e. 1,024 tokens, with the callers' settings). Selection blocks of 256 tokens
+// are left to the search.
+bool every_row_full(const fp_problem* p, const fp_ws_layout& L) {
+  const int64_t rules = static_cast<int64_t>(std::max(p->attention_sink, 0)) +
+                        std::max(p->window_size, 0) + std::max(p->last_n_block, 0);
+  return block_ratio(p) == 1 && L.nb_max <= rules;
+}
+
+// Everything of a whole-operator call before the attention. At most
+// kSmallPlanBatch sequences plan and pool in one launch (k_plan_pool), where the
+// plan's own launch and latency are a visible part of a short call, and write the
+// selection there too when it does not depend on the scores: a 1K call then has
+// two launches instead of three (39.8 -> 33 us, 32 q / 8 kv heads; the search
+// alone took 7).
+int run_before_attention(const fp_problem* p, const fp_ws_layout& L, void* ws, hipStream_t s) {
+  int rc;
+  if (p->batch <= fp::kSmallPlanBatch) {
+    const fp::SearchArgs sa = search_args(p, L, ws);
+    const fp::FullRowsArgs f = {every_row_full(p, L) ? 1 : 0, sa.Hq, sa.idx, sa.cnt, sa.rowrec,
+                                sa.tri_cap};
+    const hipError_t e = fp::launch_plan_pool(plan_args(p, L, ws), pool_args(p, L, ws), f, p->dtype,
+                                              p->head_dim, s);
+    if (e != hipSuccess) return hip_fail(e, "plan + pool launch");
+    if (f.on) return FP_OK;
+  } else {
+    if ((rc = run_plan(p, L, ws, s)) != FP_OK) return rc;
+    if ((rc = run_pool(p, L, ws, s)) != FP_OK) return rc;
+  }
+  return run_search(p, L, ws, nullptr, nullptr, nullptr, nullptr, s);
 }
 
 int run_attn(const fp_problem* p, const fp_ws_layout& L, void* ws, hipStream_t s) {
@@ -630,8 +651,7 @@ int fp_flashprefill(const fp_problem* p, void* ws, void* stream) {
   int rc = prepare(p, ws, &L);
   if (rc != FP_OK) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if ((rc = run_plan_and_pool(p, L, ws, s)) != FP_OK) return rc;
-  if ((rc = run_search(p, L, ws, nullptr, nullptr, nullptr, nullptr, s)) != FP_OK) return rc;
+  if ((rc = run_before_attention(p, L, ws, s)) != FP_OK) return rc;
   return run_attn(p, L, ws, s);
 }
 
@@ -647,8 +667,7 @@ int fp_flashprefill_noalloc(const fp_problem* p, void* stream) {
   void* ws = nullptr;
   if ((rc = scratch_on_current_device(&ws)) != FP_OK) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if ((rc = run_plan_and_pool(p, L, ws, s)) != FP_OK) return rc;
-  if ((rc = run_search(p, L, ws, nullptr, nullptr, nullptr, nullptr, s)) != FP_OK) return rc;
+  if ((rc = run_before_attention(p, L, ws, s)) != FP_OK) return rc;
   return run_attn(p, L, ws, s);
 }
 

@@ -39,6 +39,17 @@ struct PoolArgs {
   int32_t ratio;  // selection blocks are ratio x block tokens (2 at block_size 256, else 1)
 };
 
+// Selection written by k_plan_pool itself, for calls whose rules alone keep
+// every block of every row (`on`): what the search would write.
+struct FullRowsArgs {
+  int32_t on;
+  int32_t Hq;
+  int32_t* idx;
+  int32_t* cnt;
+  int32_t* rowrec;
+  int64_t tri_cap;
+};
+
 struct SearchArgs {
   SeqTables tab;
   const uint16_t* q;
@@ -183,8 +194,8 @@ hipError_t launch_paged(const PagedArgs& a, int dtype, int head_dim, int64_t til
 hipError_t launch_kv_cache_write(const KvCacheArgs& a, hipStream_t s);
 hipError_t launch_pool(const PoolArgs& a, int dtype, int head_dim, int64_t grid, hipStream_t s);
 // k_plan then k_pool as one launch (batch <= kSmallPlanBatch)
-hipError_t launch_plan_pool(const PlanArgs& pa, const PoolArgs& a, int dtype, int head_dim,
-                            hipStream_t s);
+hipError_t launch_plan_pool(const PlanArgs& pa, const PoolArgs& a, const FullRowsArgs& f, int dtype,
+                            int head_dim, hipStream_t s);
 hipError_t launch_search(const SearchArgs& a, int dtype, int head_dim, int block, int64_t grid,
                          bool from_scores, hipStream_t s);
 hipError_t launch_attn(const AttnArgs& a, int dtype, int head_dim, int block, int64_t grid,

@@ -444,6 +444,17 @@ __device__ void small_plan_table(const PlanArgs& a, SmallPlan& sp) {
   }
 }
 
+// position of row i of sequence b among the work items: after every item of a
+// higher level and after the items of its level of the sequences before b
+__device__ __forceinline__ int64_t small_plan_pos(const SmallPlan& sp, int B, int b, int i) {
+  int64_t pos = 0;
+  for (int x = 0; x < B; ++x) {
+    pos += max(sp.nb[x] - 1 - i, 0);
+    if (x < b && sp.nb[x] > i) ++pos;
+  }
+  return pos;
+}
+
 // workgroup 0 of k_plan_pool: everything k_plan writes
 __device__ void small_plan_write(const PlanArgs& a, const SmallPlan& sp) {
   const int t = threadIdx.x, B = a.B;
@@ -462,18 +473,13 @@ __device__ void small_plan_write(const PlanArgs& a, const SmallPlan& sp) {
   }
   if (t < kQueueWords) a.units[kQueueOff + t] = 0;  // empty attention work queues
   for (int64_t x = t; x < a.n_arrivals; x += blockDim.x) a.arrivals[x] = 0;
-  // work items: item (b, i) goes after every item of a higher level and
-  // after the items of level i of the sequences before b
+  // work items (small_plan_pos)
   const int64_t nsum = sp.tile[B];
   for (int64_t g = t; g < nsum; g += blockDim.x) {
     int b = 0;
     while (b + 1 < B && sp.tile[b + 1] <= g) ++b;
     const int i = static_cast<int>(g - sp.tile[b]);
-    int64_t pos = 0;
-    for (int x = 0; x < B; ++x) {
-      pos += max(sp.nb[x] - 1 - i, 0);
-      if (x < b && sp.nb[x] > i) ++pos;
-    }
+    const int64_t pos = small_plan_pos(sp, B, b, i);
     ItemRec r;
     r.b = b;
     r.i = i;
@@ -513,7 +519,7 @@ __device__ void small_plan_write(const PlanArgs& a, const SmallPlan& sp) {
 // the pooling (as the grid's last workgroup it started only once a pooling
 // slot freed up; 4K call -1.4 %, 128K unchanged).
 template <typename T, int D>
-__global__ __launch_bounds__(256) void k_plan_pool(PlanArgs pa, PoolArgs a) {
+__global__ __launch_bounds__(256) void k_plan_pool(PlanArgs pa, PoolArgs a, FullRowsArgs f) {
   __shared__ SmallPlan sp;
   if (threadIdx.x < 64) small_plan_table(pa, sp);
   __syncthreads();
@@ -529,6 +535,20 @@ __global__ __launch_bounds__(256) void k_plan_pool(PlanArgs pa, PoolArgs a) {
   while (b + 1 < a.B && sp.tile[b + 1] <= g) ++b;
   const int i = static_cast<int>(g - sp.tile[b]);
   if (i % a.ratio) return;
+  if (f.on) {
+    // row i of the query heads of kv head hh keeps blocks 0 .. i: its list,
+    // count and record (count, first two entries, diagonal kept)
+    const int G = f.Hq / a.Hkv, t = threadIdx.x;
+    const int64_t tri = sp.tri[b] + static_cast<int64_t>(i) * (i + 1) / 2;
+    for (int x = t; x < G * (i + 1); x += 256)
+      f.idx[(hh * G + x / (i + 1)) * f.tri_cap + tri + x % (i + 1)] = x % (i + 1);
+    for (int x = t; x < G; x += 256) {
+      const int64_t row = static_cast<int64_t>(hh * G + x) * a.nb_sum_cap;
+      f.cnt[row + g] = i + 1;
+      reinterpret_cast<int4*>(f.rowrec)[row + small_plan_pos(sp, a.B, b, i)] =
+          make_int4(i + 1, 0, i > 0 ? 1 : 0, 1);
+    }
+  }
   pool_block<T, D>(a, g, hh, sp.start[b] + static_cast<int64_t>(i) * a.block,
                    min(a.block * a.ratio, sp.len[b] - i * a.block));
 }
@@ -545,19 +565,19 @@ hipError_t launch_plan(const PlanArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_plan_pool(const PlanArgs& pa, const PoolArgs& a, int dtype, int head_dim,
-                            hipStream_t s) {
+hipError_t launch_plan_pool(const PlanArgs& pa, const PoolArgs& a, const FullRowsArgs& f, int dtype,
+                            int head_dim, hipStream_t s) {
   // one workgroup per (key block, kv head) of the capacity, plus the table writer
   const dim3 g(static_cast<unsigned>(a.nb_sum_cap * a.Hkv + 1)), blk(256);
   if (dtype == FP_DTYPE_F32) {  // head_dim 64 or 128
-    if (head_dim == 128) hipLaunchKernelGGL((k_plan_pool<F32, 128>), g, blk, 0, s, pa, a);
-    else hipLaunchKernelGGL((k_plan_pool<F32, 64>), g, blk, 0, s, pa, a);
+    if (head_dim == 128) hipLaunchKernelGGL((k_plan_pool<F32, 128>), g, blk, 0, s, pa, a, f);
+    else hipLaunchKernelGGL((k_plan_pool<F32, 64>), g, blk, 0, s, pa, a, f);
     return hipGetLastError();
   }
   with_head_dim(head_dim, [&](auto dc) {
     constexpr int D = decltype(dc)::value;
-    if (dtype == FP_DTYPE_BF16) hipLaunchKernelGGL((k_plan_pool<BF16, D>), g, blk, 0, s, pa, a);
-    else hipLaunchKernelGGL((k_plan_pool<F16, D>), g, blk, 0, s, pa, a);
+    if (dtype == FP_DTYPE_BF16) hipLaunchKernelGGL((k_plan_pool<BF16, D>), g, blk, 0, s, pa, a, f);
+    else hipLaunchKernelGGL((k_plan_pool<F16, D>), g, blk, 0, s, pa, a, f);
     return 0;
   });
   return hipGetLastError();
