@@ -235,6 +235,12 @@ fp::SeqTables tables(const fp_ws_layout& L, void* ws) {
   return t;
 }
 
+// Workgroups of the attention kernel per CU: waves per SIMD x 4 SIMDs / waves per
+// workgroup.
+int64_t resident_per_cu(int block, int head_dim) {
+  return (head_dim == 256 ? 4 : head_dim == 64 ? 12 : 8) / (block / 32);
+}
+
 // Workgroups of the attention kernel resident on the current device at once:
 // two per CU at block 128 (64 KB of LDS, 4 waves), four at block 64 (32 KB,
 // 2 waves), half that at d = 256 (one wave per SIMD, twice the LDS), half as
@@ -256,9 +262,7 @@ int resident_attn_workgroups(int block, int head_dim, int64_t* out) {
     if (n < 1) return fail(FP_E_LAUNCH, "device reports %d CUs", n);
     cus[dev] = n;
   }
-  // waves per SIMD x 4 SIMDs / waves per workgroup
-  const int64_t per_cu = (head_dim == 256 ? 4 : head_dim == 64 ? 12 : 8) / (block / 32);
-  *out = (cus[dev] * per_cu + 7) / 8 * 8;
+  *out = (cus[dev] * resident_per_cu(block, head_dim) + 7) / 8 * 8;
   return FP_OK;
 }
 
@@ -472,7 +476,15 @@ int run_attn(const fp_problem* p, const fp_ws_layout& L, void* ws, hipStream_t s
     if (rc != FP_OK) return rc;
     const bool persist = a.total_slots >= 4 * resident;
     const int64_t grid = persist ? resident : a.total_slots;
-    e = fp::launch_attn(a, p->dtype, p->head_dim, blk, grid, persist, s);
+    // At most one workgroup per CU: two wave groups per row (k_attn_pair), from
+    // rows of 6 blocks on (attention alone, one group -> two, d = 128: 8 blocks x
+    // 32 heads 26.9 -> 24.9 us, 32 x 4 heads 43.9 -> 40.1, 16 x 8 heads 30.9 ->
+    // 30.5; 4 blocks x 32 heads 16.5 -> 16.6, where joining the two takes what
+    // the shorter walk saves).
+    const bool pair = p->head_dim <= 128 && L.nb_max >= 6 &&
+                      a.total_slots * resident_per_cu(blk, p->head_dim) <= resident;
+    e = pair ? fp::launch_attn_pair(a, p->dtype, p->head_dim, blk, s)
+             : fp::launch_attn(a, p->dtype, p->head_dim, blk, grid, persist, s);
   }
   if (e == hipSuccess && L.split_blocks > 0 && !a.merge_inline)
     e = fp::launch_merge(a, p->dtype, p->head_dim, blk, s);
