@@ -83,6 +83,7 @@ class FpRopeArgs(ctypes.Structure):
         ("q_norm", ctypes.c_void_p), ("k_norm", ctypes.c_void_p), ("eps", ctypes.c_float),
         ("num_q_heads", ctypes.c_int32), ("num_kv_heads", ctypes.c_int32),
         ("head_dim", ctypes.c_int32), ("dtype", ctypes.c_int32),
+        ("cu_seqlens", ctypes.c_void_p), ("batch", ctypes.c_int32),
     ]
 
 

@@ -76,19 +76,27 @@ def rope_position_tables(num_positions: int, head_dim: int, theta: float, device
     return hit
 
 
-def fused_rope_qk(q: torch.Tensor, k: torch.Tensor, positions: torch.Tensor, theta: float,
+def fused_rope_qk(q: torch.Tensor, k: torch.Tensor, positions: Optional[torch.Tensor],
+                  theta: float,
                   q_norm: Optional[torch.Tensor] = None, k_norm: Optional[torch.Tensor] = None,
-                  eps: float = 1e-6, max_position: Optional[int] = None) -> None:
+                  eps: float = 1e-6, max_position: Optional[int] = None,
+                  cu_seqlens: Optional[torch.Tensor] = None) -> None:
     """RMSNorm (when the weights are given) and RoPE of q (T, Hq, d) and k
     (T, Hkv, d) in place with the HIP kernel (bf16 / fp16 on the GPU; no
-    fallback). ``positions`` (T,) int64 on the same device."""
+    fallback). ``positions`` (T,) int64 on the same device, or None with
+    ``cu_seqlens`` (B + 1,) contiguous int32 there, 1 <= B <= 64, and
+    ``max_position``: each token's place in its packed sequence."""
     T, Hq, d = q.shape
     n = int(max_position) if max_position is not None else int(positions.max().item()) + 1
     cos, sin = rope_position_tables(max(n, 1), d, theta, q.device)
     a = _lib.FpRopeArgs()
     a.q, a.q_stride_tok, a.q_stride_head = q.data_ptr(), q.stride(0), q.stride(1)
     a.k, a.k_stride_tok, a.k_stride_head = k.data_ptr(), k.stride(0), k.stride(1)
-    a.positions, a.num_tokens = positions.data_ptr(), T
+    a.num_tokens = T
+    if positions is not None:
+        a.positions = positions.data_ptr()
+    else:
+        a.cu_seqlens, a.batch = cu_seqlens.data_ptr(), cu_seqlens.numel() - 1
     a.cos_table, a.sin_table, a.num_positions = cos.data_ptr(), sin.data_ptr(), cos.shape[0]
     a.q_norm = q_norm.data_ptr() if q_norm is not None else None
     a.k_norm = k_norm.data_ptr() if k_norm is not None else None
@@ -144,15 +152,19 @@ class PrefillAttention(torch.nn.Module):
         q = qkv[:, :self.Hq]
         k = qkv[:, self.Hq:self.Hq + self.Hkv]
         v = qkv[:, self.Hq + self.Hkv:]
-        pos = positions_from_cu_seqlens(cu_seqlens, T)
         if qkv.is_cuda and qkv.dtype in (torch.bfloat16, torch.float16):
-            # one kernel, in place on the projection (q and k stay views of it)
-            fused_rope_qk(q, k, pos, self.rope_theta,
+            # one kernel, in place on the projection (q and k stay views of it);
+            # it takes the offsets of up to 64 sequences as they are
+            direct = (cu_seqlens.dtype == torch.int32 and cu_seqlens.device == qkv.device
+                      and cu_seqlens.dim() == 1 and cu_seqlens.is_contiguous()
+                      and 2 <= cu_seqlens.numel() <= 65)
+            fused_rope_qk(q, k, None if direct else positions_from_cu_seqlens(cu_seqlens, T),
+                          self.rope_theta,
                           self.q_norm if self.qk_norm else None,
                           self.k_norm if self.qk_norm else None, self.rms_eps,
-                          max_position=T)
+                          max_position=T, cu_seqlens=cu_seqlens if direct else None)
             return q, k, v
-        return self.project_qkv_reference(q, k, v, pos)
+        return self.project_qkv_reference(q, k, v, positions_from_cu_seqlens(cu_seqlens, T))
 
     def project_qkv_reference(self, q, k, v, pos):
         """The torch composition of the same steps (the fused kernel's

@@ -692,9 +692,11 @@ int fp_rope_qk(const fp_rope_args* a, void* stream) {
   if (a->num_tokens < 0 || a->num_q_heads < 0 || a->num_kv_heads < 0 || a->num_positions < 1)
     return fail(FP_E_INVALID_ARG, "rope: negative sizes or an empty table");
   if (a->num_tokens == 0) return FP_OK;
-  if ((a->num_q_heads > 0 && !a->q) || (a->num_kv_heads > 0 && !a->k) || !a->positions ||
-      !a->cos_table || !a->sin_table)
+  if ((a->num_q_heads > 0 && !a->q) || (a->num_kv_heads > 0 && !a->k) ||
+      (!a->positions && !a->cu_seqlens) || !a->cos_table || !a->sin_table)
     return fail(FP_E_INVALID_ARG, "rope: NULL pointer");
+  if (!a->positions && (a->batch < 1 || a->batch > fp::kRopeMaxBatch))
+    return fail(FP_E_INVALID_ARG, "rope: batch %d outside [1, %d]", a->batch, fp::kRopeMaxBatch);
   const int64_t st[4] = {a->q_stride_tok, a->q_stride_head, a->k_stride_tok, a->k_stride_head};
   for (int i = 0; i < 4; ++i)
     if (st[i] < 0 || st[i] % 8)
@@ -713,6 +715,10 @@ int fp_rope_qk(const fp_rope_args* a, void* stream) {
   r.num_kv_heads = a->num_kv_heads;
   r.head_dim = a->head_dim;
   r.positions = a->positions;
+  // (read only when asked for: callers with positions may pass the struct as it
+  // was before these two fields)
+  r.cu = a->positions ? nullptr : a->cu_seqlens;
+  r.batch = a->positions ? 0 : a->batch;
   r.num_tokens = a->num_tokens;
   r.cos_tab = a->cos_table;
   r.sin_tab = a->sin_table;

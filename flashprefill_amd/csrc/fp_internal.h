@@ -161,13 +161,17 @@ struct PagedArgs {
   float* ml;         // [T * Hq][nc] (m, l) pairs
 };
 
+constexpr int kRopeMaxBatch = 64;  // sequences whose offsets k_rope takes
+
 struct RopeArgs {
   void* q;
   int64_t q_stride_tok, q_stride_head;
   void* k;
   int64_t k_stride_tok, k_stride_head;
   int32_t num_q_heads, num_kv_heads, head_dim;
-  const int64_t* positions;  // per token
+  const int64_t* positions;  // per token, or null:
+  const int32_t* cu;         // the packed sequences' offsets, batch of them
+  int32_t batch;
   int64_t num_tokens;
   const float* cos_tab;      // (num_positions, head_dim / 2)
   const float* sin_tab;

@@ -247,7 +247,9 @@ int fp_paged_attention(const fp_paged_args* a, void* workspace, void* stream);
  *   x <- round(x * rsqrt(mean(x^2) + eps) * norm)   when the head's norm is set
  *   x[j]       <- round(x[j] * cos[p][j] - x[j + d/2] * sin[p][j])
  *   x[j + d/2] <- round(x[j + d/2] * cos[p][j] + x[j] * sin[p][j]),  j < d/2,
- * p = positions[t] (clamped to the table), fp32 math, each product and sum
+ * p = positions[t], or with positions NULL the token's place in its sequence by
+ * cu_seqlens (batch ascending offsets from 0; at most 64 sequences), clamped to
+ * the table; fp32 math, each product and sum
  * rounded on its own (the bits of the torch composition of the same steps).
  * Strides in elements (multiples of 8), head dim contiguous. */
 typedef struct fp_rope_args {
@@ -255,7 +257,7 @@ typedef struct fp_rope_args {
     int64_t q_stride_tok, q_stride_head;
     void* k;                  /* (tokens, num_kv_heads, head_dim), updated in place */
     int64_t k_stride_tok, k_stride_head;
-    const int64_t* positions; /* device, num_tokens entries */
+    const int64_t* positions; /* device, num_tokens entries; NULL: cu_seqlens */
     int64_t num_tokens;
     const float* cos_table;   /* device fp32 (num_positions, head_dim / 2) */
     const float* sin_table;
@@ -267,6 +269,8 @@ typedef struct fp_rope_args {
     int32_t num_kv_heads;
     int32_t head_dim;         /* 64, 128 or 256 */
     int32_t dtype;            /* FP_DTYPE_BF16 or FP_DTYPE_F16 */
+    const int32_t* cu_seqlens; /* device, `batch` entries, read when positions is NULL */
+    int32_t batch;
 } fp_rope_args;
 int fp_rope_qk(const fp_rope_args* a, void* stream);
 
