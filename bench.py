@@ -25,7 +25,7 @@ if ROOT not in sys.path:
 
 METRIC = ("128K prefill attn latency (ms) + effective TFLOPS, speedup vs dense at 1 MI355X")
 PEAK_BF16_TFLOPS = 2500.0   # MI355X dense bf16 MFMA
-PEAK_FP32_TFLOPS = 157.3    # MI355X dense fp32 MFMA (config 1 runs fp32 inputs)
+PEAK_FP32_TFLOPS = 157.3    # MI355X dense fp32 MFMA (scale of the fp32 input config)
 PEAK_HBM_GBPS = 8000.0
 MAX_GFX_MHZ = 2400.0         # MI355X shader clock ceiling (amd-smi gfx max_clk); the bf16 peak is quoted at it
 
@@ -602,9 +602,9 @@ def config1_report(args):
         gpu_call()
         gpu_ms = timed(gpu_call, 20)
         err = (od[0].cpu() - res.out[0]).abs()
-        # the attention stage alone (fp32 MFMA kernel) on the same input in
-        # the batched layout: executed block FLOPs / its time, against the
-        # fp32 MFMA peak
+        # the attention stage alone on the same input in the batched layout:
+        # executed block FLOPs / its time, against the fp32 MFMA peak (the
+        # kernel forms its fp32 products on the bf16 units from exact parts)
         from flashprefill_amd.runtime import FlashPrefillCall
         call = FlashPrefillCall(qd[0], kd[0], vd[0], torch.empty_like(qd[0]), None, S,
                                 alpha=args.alpha, attention_sink=2, window_size=4,

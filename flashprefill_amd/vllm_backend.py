@@ -39,10 +39,10 @@ from dataclasses import dataclass
 from typing import Any, Callable, Dict, Optional
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 from .flashprefill_varlen_func import flash_prefill_varlen_func
-from .runtime import WORKSPACES
 
 # Per-model selection configs of the reference patch
 # (patches/patch_loader_vllm_0_12_0.py:13-40): block 128, sink 2, window 4,
@@ -137,8 +137,11 @@ def _rows_ok(t: torch.Tensor) -> bool:
 def _paged_kernel_takes(query, key_cache, value_cache, out, cu, used, table) -> bool:
     """Whether the HIP kernels take this call as it is: 16-bit tensors of one
     type on one GPU, head_dim 64 / 128 / 256, 16-byte aligned rows, int32 /
-    int64 metadata of matching shapes."""
+    int64 metadata of matching shapes, no derivative or functional transform
+    to carry along (dual numbers and vmap see only torch operations)."""
     if not query.is_cuda or query.dtype not in _DTYPES:
+        return False
+    if forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None:
         return False
     dev, dt = query.device, query.dtype
     if query.dim() != 3 or out.dim() != 3 or key_cache.dim() != 4 or \
@@ -190,7 +193,11 @@ def _paged_attention_kernel(query, key_cache, value_cache, out, cu, used, table,
     a.softmax_scale = float(scale)
     lib = _lib.load()
     with torch.cuda.device(dev):
-        ws = WORKSPACES.get(dev, max(int(lib.fp_paged_workspace_bytes(ctypes.byref(a))), 256))
+        # A buffer of this call's own: threads that share a stream may interleave
+        # their launches, and a shared one would be written between the chunks and
+        # their merge. The caching allocator hands it on in stream order.
+        ws = torch.empty(max(int(lib.fp_paged_workspace_bytes(ctypes.byref(a))), 256),
+                         dtype=torch.uint8, device=dev)
         _lib.check(lib.fp_paged_attention(ctypes.byref(a), ws.data_ptr(),
                                           torch.cuda.current_stream(dev).cuda_stream))
 

@@ -48,7 +48,7 @@ extern "C" {
 
 #define FP_DTYPE_BF16 0
 #define FP_DTYPE_F16 1
-#define FP_DTYPE_F32 2  /* fp32 kernels (fp32 MFMA); pooled K is fp32 in the workspace */
+#define FP_DTYPE_F32 2  /* fp32 kernels; pooled K is fp32 in the workspace */
 
 /* Device-side status flags (`fp_status` word in the workspace, see
  * fp_read_status): set by the kernels when cu_seqlens disagrees with the host

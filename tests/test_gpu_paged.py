@@ -185,3 +185,52 @@ def test_capture_and_replay():
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+
+
+def test_threads_on_one_stream():
+    """Two threads on the default stream, chunked calls: neither's partial sums
+    reach the other's merge."""
+    import threading
+
+    cases = [_case([3000 + 500 * i, 700], [1, 1], 8, 2, 128, 16, torch.bfloat16, seed=60 + i)
+             for i in range(2)]
+    dev = [[t.to(DEV) for t in c] for c in cases]
+    scale = 1 / math.sqrt(128)
+    want, got = [], [[], []]
+    for c in dev:
+        out = torch.empty_like(c[0])
+        vb.paged_decode_attention(c[0], c[1], c[2], out, *c[3:], scale)
+        want.append(out.clone())
+
+    def work(i):
+        c = dev[i]
+        for _ in range(200):
+            out = torch.empty_like(c[0])
+            vb.paged_decode_attention(c[0], c[1], c[2], out, *c[3:], scale)
+            got[i].append(out)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert len(got[i]) == 200 and all(torch.equal(o, want[i]) for o in got[i])
+
+
+def test_forward_mode_keeps_its_tangent():
+    """Dual numbers take the torch composition, which carries the tangent: the
+    derivative of the output in the values is the attention of the tangent."""
+    from torch.autograd import forward_ad
+
+    q, kc, vc, cu, used, table = [t.to(DEV) for t in
+                                  _case([48, 32], [1, 1], 8, 2, 64, 16, torch.bfloat16, spare=0)]
+    tv = torch.randn(vc.shape, device=DEV).to(vc.dtype)
+    want, out = torch.empty_like(q), torch.zeros_like(q)
+    vb.paged_attention_reference(q, kc, tv, want, cu, used, table, 0.125)
+    with forward_ad.dual_level():
+        vb.paged_decode_attention(q, kc, forward_ad.make_dual(vc, tv), out, cu, used, table, 0.125)
+        tangent = forward_ad.unpack_dual(out).tangent
+        assert tangent is not None
+        assert torch.equal(tangent, want)
