@@ -517,8 +517,10 @@ __device__ void small_plan_write(const PlanArgs& a, const SmallPlan& sp) {
 
 // Workgroup 0 writes the tables and items: dispatched first, it runs beside
 // the pooling (as the grid's last workgroup it started only once a pooling
-// slot freed up; 4K call -1.4 %, 128K unchanged).
-template <typename T, int D>
+// slot freed up; 4K call -1.4 %, 128K unchanged). FULL: the call's rules alone
+// decide the selection, which is written here too (a variant of its own: a branch
+// inside the one kernel took 32K x 8 KV heads from 18.0 to 21.5 us).
+template <typename T, int D, bool FULL>
 __global__ __launch_bounds__(256) void k_plan_pool(PlanArgs pa, PoolArgs a, FullRowsArgs f) {
   __shared__ SmallPlan sp;
   if (threadIdx.x < 64) small_plan_table(pa, sp);
@@ -535,7 +537,7 @@ __global__ __launch_bounds__(256) void k_plan_pool(PlanArgs pa, PoolArgs a, Full
   while (b + 1 < a.B && sp.tile[b + 1] <= g) ++b;
   const int i = static_cast<int>(g - sp.tile[b]);
   if (i % a.ratio) return;
-  if (f.on) {
+  if constexpr (FULL) {
     // row i of the query heads of kv head hh keeps blocks 0 .. i: its list,
     // count and record (count, first two entries, diagonal kept)
     const int G = f.Hq / a.Hkv, t = threadIdx.x;
@@ -569,16 +571,20 @@ hipError_t launch_plan_pool(const PlanArgs& pa, const PoolArgs& a, const FullRow
                             int head_dim, hipStream_t s) {
   // one workgroup per (key block, kv head) of the capacity, plus the table writer
   const dim3 g(static_cast<unsigned>(a.nb_sum_cap * a.Hkv + 1)), blk(256);
+  const auto run = [&](auto type, auto dc) {
+    typedef decltype(type) T;
+    constexpr int D = decltype(dc)::value;
+    if (f.on) hipLaunchKernelGGL((k_plan_pool<T, D, true>), g, blk, 0, s, pa, a, f);
+    else hipLaunchKernelGGL((k_plan_pool<T, D, false>), g, blk, 0, s, pa, a, f);
+    return 0;
+  };
   if (dtype == FP_DTYPE_F32) {  // head_dim 64 or 128
-    if (head_dim == 128) hipLaunchKernelGGL((k_plan_pool<F32, 128>), g, blk, 0, s, pa, a, f);
-    else hipLaunchKernelGGL((k_plan_pool<F32, 64>), g, blk, 0, s, pa, a, f);
+    if (head_dim == 128) run(F32(), std::integral_constant<int, 128>());
+    else run(F32(), std::integral_constant<int, 64>());
     return hipGetLastError();
   }
   with_head_dim(head_dim, [&](auto dc) {
-    constexpr int D = decltype(dc)::value;
-    if (dtype == FP_DTYPE_BF16) hipLaunchKernelGGL((k_plan_pool<BF16, D>), g, blk, 0, s, pa, a, f);
-    else hipLaunchKernelGGL((k_plan_pool<F16, D>), g, blk, 0, s, pa, a, f);
-    return 0;
+    return dtype == FP_DTYPE_BF16 ? run(BF16(), dc) : run(F16(), dc);
   });
   return hipGetLastError();
 }
