@@ -234,3 +234,12 @@ def test_forward_mode_keeps_its_tangent():
         tangent = forward_ad.unpack_dual(out).tangent
         assert tangent is not None
         assert torch.equal(tangent, want)
+
+
+@pytest.mark.parametrize("hq,hkv", [(1, 1), (5, 5), (6, 3), (7, 1), (9, 3)])
+@pytest.mark.parametrize("d", [64, 128])
+def test_merge_of_many_rows_at_head_counts(hq, hkv, d):
+    """Head counts that are no multiple of the merge's four heads per wave, with
+    sequences of one, two and several chunks and one of no query."""
+    _check(_case([1300, 70, 700, 40], [41, 33, 35, 0], hq, hkv, d, 16, torch.bfloat16),
+           1 / math.sqrt(d))
