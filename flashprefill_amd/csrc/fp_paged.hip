@@ -518,7 +518,7 @@ __device__ __forceinline__ void part_pair(float x0, float x1, uint32_t (&u)[3]) 
 // fp32: P.V runs on its three exact 16-bit parts (48 of the 64 MFMAs of a tile
 // and wave at d = 128). Bound by these MFMAs and the instructions that form the
 // parts. Measured (one MI355X): 500 new tokens each on 6,144, 2,500 and 1,111
-// cached ones (28 q / 4 kv heads, d = 128) 504 us with k_paged, 182 here; 4 x
+// cached ones (28 q / 4 kv heads, d = 128) 504 us with k_paged, 172 here; 4 x
 // 2,048 new of 4,096 (32 q / 8 kv) 3,045 -> 890 us = 463 TFLOP/s (924 of MFMAs).
 template <typename T, int D, bool P16>
 __global__ __launch_bounds__(256, 2) void k_paged_rows(PagedArgs a) {
