@@ -903,8 +903,15 @@ __device__ __forceinline__ bool attn_slot(const Args& a, int slot, int t, Tail t
   __shared__ alignas(D > 128 ? 1024 : 16) uint4 skv[GROUPS][2][BLK * CH];
   const int grp = GROUPS == 1 ? 0 : __builtin_amdgcn_readfirstlane(t / (64 * NW));
   if constexpr (GROUPS > 1) t &= 64 * NW - 1;
-  uint4* const sk = skv[grp][0];
-  uint4* const sv = skv[grp][1];
+  uint4 *sk = skv[grp][0], *sv = skv[grp][1];
+  if constexpr (GROUPS == 1 && D <= 128) {
+    // two arrays of their own (skv is not allocated then): as halves of one, the
+    // rows' address setup came out longer and the prefill 0.3 % slower
+    __shared__ uint4 sk1[BLK * CH];
+    __shared__ uint4 sv1[BLK * CH];
+    sk = sk1;
+    sv = sv1;
+  }
 
   // Work item: the first unit_slots slots take the chunks of the split
   // rows (a slice of a dense row's list, fp32 partials out), the others one
