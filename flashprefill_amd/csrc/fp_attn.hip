@@ -25,13 +25,4 @@ hipError_t launch_attn(const AttnArgs& a, int dtype, int head_dim, int block, in
                                 : launch_attn_t<F16, 64>(a, block, grid, persist, s);
 }
 
-hipError_t launch_attn_pair(const AttnArgs& a, int dtype, int head_dim, int block, hipStream_t s) {
-  if (a.total_slots <= 0) return hipSuccess;
-  if (head_dim == 128)
-    return dtype == FP_DTYPE_BF16 ? launch_attn_pair_t<BF16, 128>(a, block, s)
-                                  : launch_attn_pair_t<F16, 128>(a, block, s);
-  return dtype == FP_DTYPE_BF16 ? launch_attn_pair_t<BF16, 64>(a, block, s)
-                                : launch_attn_pair_t<F16, 64>(a, block, s);
-}
-
 }  // namespace fp

@@ -886,13 +886,7 @@ __device__ __forceinline__ void merge_if_last(const Args& a, int h, int u0, int 
 // once the slot's last block is done, before the output is normalised and
 // stored (the persistent grid claims its next slot there, so the claim's
 // latency passes behind the stores); returns whether it ran.
-//
-// GROUPS = 2 (k_attn_pair): two groups of BLK / 32 waves with K and V buffers of
-// their own walk the even and the odd entries of the row's list; group 1 then
-// leaves its O, m and l in LDS and group 0 adds them to its own and finishes the
-// row. The groups run through the same workgroup barriers, so the one with fewer
-// blocks makes up the count.
-template <typename T, int D, int BLK, int GROUPS, typename Args, typename Tail>
+template <typename T, int D, int BLK, typename Args, typename Tail>
 __device__ __forceinline__ bool attn_slot(const Args& a, int slot, int t, Tail tail) {
   constexpr int CH = D / 8;   // 16-byte chunks per row
   constexpr int KS = D / 16;  // MFMA k-steps over the head dim
@@ -900,18 +894,8 @@ __device__ __forceinline__ bool attn_slot(const Args& a, int slot, int t, Tail t
   constexpr int NW = BLK / 32;
   // (d = 256: aligned to whole rows, operand addresses are formed by exclusive
   // or of chunk bits)
-  __shared__ alignas(D > 128 ? 1024 : 16) uint4 skv[GROUPS][2][BLK * CH];
-  const int grp = GROUPS == 1 ? 0 : __builtin_amdgcn_readfirstlane(t / (64 * NW));
-  if constexpr (GROUPS > 1) t &= 64 * NW - 1;
-  uint4 *sk = skv[grp][0], *sv = skv[grp][1];
-  if constexpr (GROUPS == 1 && D <= 128) {
-    // two arrays of their own (skv is not allocated then): as halves of one, the
-    // rows' address setup came out longer and the prefill 0.3 % slower
-    __shared__ uint4 sk1[BLK * CH];
-    __shared__ uint4 sv1[BLK * CH];
-    sk = sk1;
-    sv = sv1;
-  }
+  __shared__ alignas(D > 128 ? 1024 : 16) uint4 sk[BLK * CH];
+  __shared__ alignas(D > 128 ? 1024 : 16) uint4 sv[BLK * CH];
 
   // Work item: the first unit_slots slots take the chunks of the split
   // rows (a slice of a dense row's list, fp32 partials out), the others one
@@ -972,15 +956,8 @@ __device__ __forceinline__ bool attn_slot(const Args& a, int slot, int t, Tail t
   const int64_t row_tri = static_cast<int64_t>(h) * a.tri_cap + rec.tri;
   const int32_t* list = a.idx + row_tri + first;
   const int kvh = h / (a.Hq / a.Hkv);
-  const int nall = ncnt;  // the row's blocks; below, this group's
-  if constexpr (GROUPS > 1) {
-    if (grp == 1) j0 = jraw;
-    jraw = sld(list + max(min(2 + grp, nall - 1), 0));
-    has_diag = has_diag && ((nall - 1) & 1) == grp;
-    ncnt = (nall + 1 - grp) / 2;
-  }
 
-  const int lane = t & 63;  // t: threadIdx.x (in the group)
+  const int lane = t & 63;  // t: threadIdx.x
   const int w = __builtin_amdgcn_readfirstlane(t >> 6);  // wave index, kept in an SGPR
   const int half = lane >> 5, l32 = lane & 31;
   const int qrow = 32 * w + l32;           // query row inside the block
@@ -1032,7 +1009,7 @@ __device__ __forceinline__ bool attn_slot(const Args& a, int slot, int t, Tail t
       qb[s] = as_vec8<T>(__builtin_bit_cast(uint4, u[s]));
     }
   }
-  if (nall > 0) vm_barrier<0>();  // the first block's K and V have landed
+  if (ncnt > 0) vm_barrier<0>();  // the first block's K and V have landed
 
   AttnState<T, D> st;
 #pragma unroll
@@ -1041,12 +1018,8 @@ __device__ __forceinline__ bool attn_slot(const Args& a, int slot, int t, Tail t
   // the two halves' partial sums add up to l: a row starts from the
   // reference's l = 1.0 (cleared by its first block's rescale, alpha =
   // exp2(-inf) = 0), a chunk of a split row from l = 0
-  st.l_part = half == 0 && unit < 0 && grp == 0 ? 1.0f : 0.0f;
+  st.l_part = half == 0 && unit < 0 ? 1.0f : 0.0f;
 
-  // group 1 stays one barrier interval behind, so that the groups' MFMAs meet the
-  // other's softmax in two of the three intervals of a block
-  if constexpr (GROUPS > 1)
-    if (grp == 1) asm volatile("s_barrier" ::: "memory");
   const uint16_t* sv16 = reinterpret_cast<const uint16_t*>(sv);
   if constexpr (D > 128) {
     f32x16 s[2][1];
@@ -1072,7 +1045,7 @@ __device__ __forceinline__ bool attn_slot(const Args& a, int slot, int t, Tail t
     const int nplain = ncnt - (has_diag ? 1 : 0);
     // block n refills the buffers with entry n + 1 and prefetches entry n + 2
     // (the last entry past the end of the list; not used then)
-    auto entry = [&](int n) { return list + min(GROUPS * n + grp, nall - 1); };
+    auto entry = [&](int n) { return list + min(n, ncnt - 1); };
     for (int n = 0; n < nplain; ++n) {
       const int jn = n + 1 < ncnt ? min(max(jraw, 0), i) : -1;
       if constexpr (D == 64 && BLK == 128) {
@@ -1094,53 +1067,6 @@ __device__ __forceinline__ bool attn_slot(const Args& a, int slot, int t, Tail t
                                     -1, list, unused, L, c, nplain == 0, w, lane);
       }
     }
-  }
-
-  if constexpr (GROUPS > 1) {
-    // m blocks pass 3 m - 1 barriers (a block's S, its V wait, and the refill
-    // between two blocks)
-    const int n0 = (nall + 1) / 2;
-    const int extra = (n0 > 0 ? 3 * n0 - 1 : 0) - (ncnt > 0 ? 3 * ncnt - 1 : 0) + (grp == 0 ? 1 : 0);
-    for (int x = 0; x < extra; ++x) asm volatile("s_barrier" ::: "memory");
-    if (nall > 1) {
-      __shared__ float sml[2][64 * NW];
-      // thread t of either group holds the same query and dims of O
-      static_assert(sizeof(st.o) * 64 * NW <= sizeof(skv[1]), "O of a group in its K and V buffers");
-      float4* so1 = reinterpret_cast<float4*>(skv[1][0]);
-      lds_barrier();  // every wave of group 1 is done with its buffers
-      if (grp == 1) {
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-          for (int g4 = 0; g4 < 4; ++g4)
-            so1[(4 * dt + g4) * 64 * NW + t] =
-                make_float4(st.o[dt][4 * g4], st.o[dt][4 * g4 + 1], st.o[dt][4 * g4 + 2],
-                            st.o[dt][4 * g4 + 3]);
-        sml[0][t] = st.m_run;
-        sml[1][t] = st.l_part;
-      }
-      lds_barrier();
-      if (grp == 0) {
-        const float m1 = sml[0][t], m = fmaxf(st.m_run, m1);
-        // NaN (-inf - -inf) counts as 1, as in the block loop
-        float f0 = __builtin_amdgcn_exp2f(st.m_run - m), f1 = __builtin_amdgcn_exp2f(m1 - m);
-        if (f0 != f0) f0 = 1.0f;
-        if (f1 != f1) f1 = 1.0f;
-        st.m_run = m;
-        st.l_part = st.l_part * f0 + sml[1][t] * f1;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-          for (int g4 = 0; g4 < 4; ++g4) {
-            const float4 y = so1[(4 * dt + g4) * 64 * NW + t];
-            st.o[dt][4 * g4] = st.o[dt][4 * g4] * f0 + y.x * f1;
-            st.o[dt][4 * g4 + 1] = st.o[dt][4 * g4 + 1] * f0 + y.y * f1;
-            st.o[dt][4 * g4 + 2] = st.o[dt][4 * g4 + 2] * f0 + y.z * f1;
-            st.o[dt][4 * g4 + 3] = st.o[dt][4 * g4 + 3] * f0 + y.w * f1;
-          }
-      }
-    }
-    if (grp == 1) return true;  // group 0 finishes the row
   }
 
   tail();
@@ -1226,7 +1152,7 @@ __global__ __launch_bounds__(2 * BLK, D > 128 ? 1 : D == 64 ? 3 : 2) void k_attn
   const __attribute__((address_space(4))) AttnArgs* ap =
       (const __attribute__((address_space(4))) AttnArgs*)__builtin_amdgcn_kernarg_segment_ptr();
   if constexpr (!PERSIST) {
-    attn_slot<T, D, BLK, 1>(*ap, static_cast<int>(blockIdx.x), static_cast<int>(threadIdx.x), [] {});
+    attn_slot<T, D, BLK>(*ap, static_cast<int>(blockIdx.x), static_cast<int>(threadIdx.x), [] {});
   } else {
     __shared__ int claim;
     const int x = static_cast<int>(blockIdx.x & 7);
@@ -1258,25 +1184,12 @@ __global__ __launch_bounds__(2 * BLK, D > 128 ? 1 : D == 64 ? 3 : 2) void k_attn
       // hoisted out of this loop, where they would stay live across it
       int t = static_cast<int>(threadIdx.x);
       asm volatile("" : "+v"(t));
-      if (!attn_slot<T, D, BLK, 1>(*ap, static_cast<int>(slot), t, claim_next)) claim_next();
+      if (!attn_slot<T, D, BLK>(*ap, static_cast<int>(slot), t, claim_next)) claim_next();
       __syncthreads();  // K / V buffers are free and `claim` is set
       slot = 8 * (g8 + claim) + x;
       __syncthreads();  // every wave has read `claim`
     }
   }
-}
-
-// k_attn without the persistent loop for grids of at most one workgroup per CU
-// (head dims 64 and 128): two groups of waves share a row (attn_slot), so that
-// a SIMD has two waves although its CU has one row. A row of 8 blocks took 2.6
-// us per block with one group; 1K tokens x 32 heads 26.9 -> 24.9 us. (With the
-// groups in step, both in the same phase of a block, 25.5; two K and two V
-// buffers for one group instead, loads a whole block ahead: 30.8.)
-template <typename T, int D, int BLK>
-__global__ __launch_bounds__(4 * BLK, 2) void k_attn_pair(AttnArgs a) {
-  const __attribute__((address_space(4))) AttnArgs* ap =
-      (const __attribute__((address_space(4))) AttnArgs*)__builtin_amdgcn_kernarg_segment_ptr();
-  attn_slot<T, D, BLK, 2>(*ap, static_cast<int>(blockIdx.x), static_cast<int>(threadIdx.x), [] {});
 }
 
 // Output rows of the split rows. Workgroup (slot, s) of the grid
@@ -1319,14 +1232,6 @@ hipError_t launch_attn_t(const AttnArgs& a, int block, int64_t grid, bool persis
     if (persist) hipLaunchKernelGGL((k_attn<T, D, 64, true>), g, dim3(128), 0, s, a);
     else hipLaunchKernelGGL((k_attn<T, D, 64, false>), g, dim3(128), 0, s, a);
   }
-  return hipGetLastError();
-}
-
-template <typename T, int D>
-hipError_t launch_attn_pair_t(const AttnArgs& a, int block, hipStream_t s) {
-  const dim3 g(static_cast<unsigned>(a.total_slots));
-  if (block == 128) hipLaunchKernelGGL((k_attn_pair<T, D, 128>), g, dim3(512), 0, s, a);
-  else hipLaunchKernelGGL((k_attn_pair<T, D, 64>), g, dim3(256), 0, s, a);
   return hipGetLastError();
 }
 

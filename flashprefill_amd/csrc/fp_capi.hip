@@ -476,15 +476,7 @@ int run_attn(const fp_problem* p, const fp_ws_layout& L, void* ws, hipStream_t s
     if (rc != FP_OK) return rc;
     const bool persist = a.total_slots >= 4 * resident;
     const int64_t grid = persist ? resident : a.total_slots;
-    // At most one workgroup per CU: two wave groups per row (k_attn_pair), from
-    // rows of 6 blocks on (attention alone, one group -> two, d = 128: 8 blocks x
-    // 32 heads 26.9 -> 24.9 us, 32 x 4 heads 43.9 -> 40.1, 16 x 8 heads 30.9 ->
-    // 30.5; 4 blocks x 32 heads 16.5 -> 16.6, where joining the two takes what
-    // the shorter walk saves).
-    const bool pair = p->head_dim <= 128 && L.nb_max >= 6 &&
-                      a.total_slots * resident_per_cu(blk, p->head_dim) <= resident;
-    e = pair ? fp::launch_attn_pair(a, p->dtype, p->head_dim, blk, s)
-             : fp::launch_attn(a, p->dtype, p->head_dim, blk, grid, persist, s);
+    e = fp::launch_attn(a, p->dtype, p->head_dim, blk, grid, persist, s);
   }
   if (e == hipSuccess && L.split_blocks > 0 && !a.merge_inline)
     e = fp::launch_merge(a, p->dtype, p->head_dim, blk, s);

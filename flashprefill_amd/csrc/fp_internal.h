@@ -206,8 +206,6 @@ hipError_t launch_attn(const AttnArgs& a, int dtype, int head_dim, int block, in
                        bool persist, hipStream_t s);
 // combines the chunk partials of the split rows into their output rows
 hipError_t launch_merge(const AttnArgs& a, int dtype, int head_dim, int block, hipStream_t s);
-// one workgroup of two wave groups per slot (head dims 64 and 128)
-hipError_t launch_attn_pair(const AttnArgs& a, int dtype, int head_dim, int block, hipStream_t s);
 // head dim 256 (fp_attn_d256.hip)
 hipError_t launch_attn_d256(const AttnArgs& a, int dtype, int block, int64_t grid, bool persist,
                             hipStream_t s);
