@@ -529,6 +529,7 @@ __global__ __launch_bounds__(256, 2) void k_paged_rows(PagedArgs a) {
   static_assert(NI * RPW == 16, "a wave loads 16 consecutive keys of a tile");
   __shared__ uint4 sk[2][KT * CH];
   __shared__ uint4 sv[2][KT * CH];
+  __shared__ int s_bad;  // some wave looked up a page outside the cache
   const int h = static_cast<int>(blockIdx.x % a.Hkv);
   const int64_t x = blockIdx.x / a.Hkv;
   const int c = static_cast<int>(blockIdx.y);
@@ -619,6 +620,8 @@ __global__ __launch_bounds__(256, 2) void k_paged_rows(PagedArgs a) {
   const int tr_row = 4 * (g16 >> 1) + (i16 >> 2);
   const int tr_col = 16 * (g16 & 1) + 4 * (i16 & 3);
 
+  // (ordered before the flag by the barrier after the loop)
+  if (t == 0) s_bad = 0;
   if (k0 < k1) issue(k0, 0);
   int buf = 0;
   for (int base = k0; base < k1; base += KT, buf ^= 1) {
@@ -711,8 +714,13 @@ __global__ __launch_bounds__(256, 2) void k_paged_rows(PagedArgs a) {
     }
   }
 
+  // A wave looks up the pages of its 16 keys of a tile only, and all four use the
+  // tile: a bad page found by one makes the rows of all four NaN.
   float l = pair32_sum(l_part);
-  if (__ballot(bad) != 0) l = __uint_as_float(0x7fc00000u);
+  lds_barrier();
+  if (bad) s_bad = 1;
+  lds_barrier();
+  if (s_bad != 0) l = __uint_as_float(0x7fc00000u);
   if (!rvalid) return;
   if (single) {
     const float rcp = 1.0f / l;

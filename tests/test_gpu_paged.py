@@ -166,6 +166,24 @@ def test_what_only_the_device_sees():
     assert torch.equal(got[1], want[1])
 
 
+@pytest.mark.parametrize("page", [16, 24, 64])
+@pytest.mark.parametrize("d,dtype", [(128, torch.bfloat16), (64, torch.float16)])
+def test_a_page_outside_the_cache_at_many_rows(page, d, dtype):
+    """40 queries per sequence share the loaded tiles: a bad page at any of the
+    tile's four 16-key positions makes every row of its sequence NaN, in several
+    chunks (1000 tokens) and in one (200); the other sequence keeps its bits."""
+    args = _case([1000, 200], [40, 40], 8, 2, d, page, dtype, seed=page)
+    want = _run(args, 0.1)
+    for b, first in ((0, 384), (1, 64)):
+        for pos in range(4):
+            t2 = args[5].clone()
+            t2[b, (first + 16 * pos) // page] = (args[1].shape[0], -args[1].shape[0] - 1)[pos % 2]
+            got = _run((*args[:5], t2), 0.1)
+            rows, rest = slice(40 * b, 40 * b + 40), slice(40 - 40 * b, 80 - 40 * b)
+            assert got[rows].isnan().all(), (b, pos, got[rows].isnan().float().mean())
+            assert torch.equal(got[rest], want[rest]), (b, pos)
+
+
 def test_capture_and_replay():
     q, kc, vc, cu, used, table = [t.to(DEV) for t in
                                   _case([900, 70], [1, 1], 8, 2, 128, 16, torch.bfloat16)]
