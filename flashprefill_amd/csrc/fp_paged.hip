@@ -714,6 +714,57 @@ __global__ __launch_bounds__(256, 2) void k_paged_rows(PagedArgs a) {
     }
   }
 
+  // An infinite or NaN value times the parts of P is NaN where its product with P
+  // is not (a part may be 0 or negative), so rows whose O is not finite take P.V
+  // again in fp32 with P whole, over the keys that each row sees; m and l hold.
+  float nf = 0.0f;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) nf = fmaf(o[dt][v], 0.0f, nf);
+  if (__ballot(nf != 0.0f) != 0) {
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) o[dt] = f32x16{};
+    const float ms = (m_run == -INFINITY ? 0.0f : m_run) - PParts<T>::kPShift;
+    // (formed here: kept live across the loop above, the offsets cost d = 64 its
+    // third wave per SIMD, 781 -> 826 us for 4 x 2,048 new of 6,144 tokens)
+    int half2 = static_cast<int>(threadIdx.x);
+    asm volatile("" : "+v"(half2));
+    half2 = (half2 >> 5) & 1;
+#pragma unroll 1
+    for (int key = k0; key < k1; ++key) {
+      const int64_t pg = paged_page<true>(a, row, key, bad);
+      const int in = key % a.bs;
+      const uint16_t* kp = kc + pg * a.kcb + static_cast<int64_t>(in) * a.kcs + 8 * half2;
+      const uint16_t* vp = vc + pg * a.vcb + static_cast<int64_t>(in) * a.vcs + 4 * half2;
+      float x = 0.0f;  // the lane's dims of q . k
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        const uint4 ku = ld16(kp + 16 * s), qu = __builtin_bit_cast(uint4, qb[s]);
+        const uint32_t kw[4] = {ku.x, ku.y, ku.z, ku.w}, qw[4] = {qu.x, qu.y, qu.z, qu.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          x = fmaf(T::to_f32(static_cast<uint16_t>(qw[e])), T::to_f32(static_cast<uint16_t>(kw[e])), x);
+          x = fmaf(T::to_f32(static_cast<uint16_t>(qw[e] >> 16)),
+                   T::to_f32(static_cast<uint16_t>(kw[e] >> 16)), x);
+        }
+      }
+      x = pair32_sum(x) * a.scale_log2;
+      if (key > lim) continue;
+      const float p = __builtin_amdgcn_exp2f(x - ms);
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4) {
+          const uint2 u = *reinterpret_cast<const uint2*>(vp + 32 * dt + 8 * g4);
+          o[dt][4 * g4] = fmaf(p, T::to_f32(static_cast<uint16_t>(u.x)), o[dt][4 * g4]);
+          o[dt][4 * g4 + 1] = fmaf(p, T::to_f32(static_cast<uint16_t>(u.x >> 16)), o[dt][4 * g4 + 1]);
+          o[dt][4 * g4 + 2] = fmaf(p, T::to_f32(static_cast<uint16_t>(u.y)), o[dt][4 * g4 + 2]);
+          o[dt][4 * g4 + 3] = fmaf(p, T::to_f32(static_cast<uint16_t>(u.y >> 16)), o[dt][4 * g4 + 3]);
+        }
+    }
+  }
+
   // A wave looks up the pages of its 16 keys of a tile only, and all four use the
   // tile: a bad page found by one makes the rows of all four NaN.
   float l = pair32_sum(l_part);

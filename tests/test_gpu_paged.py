@@ -261,3 +261,37 @@ def test_merge_of_many_rows_at_head_counts(hq, hkv, d):
     sequences of one, two and several chunks and one of no query."""
     _check(_case([1300, 70, 700, 40], [41, 33, 35, 0], hq, hkv, d, 16, torch.bfloat16),
            1 / math.sqrt(d))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("news", [1, 40])
+@pytest.mark.parametrize("d,page", [(128, 16), (64, 24)])
+def test_infinite_values(dtype, news, d, page):
+    """+inf and -inf in V at keys that every row sees: those dims are infinite, the
+    others what they are without; in several chunks and in one."""
+    lens = [1000, 200]
+    args = _case(lens, [news] * 2, 8, 2, d, page, dtype, seed=3)
+    scale = 1 / math.sqrt(d)
+    for b, key in ((0, 500), (1, 77)):
+        at = int(args[5][b, key // page]), key % page
+        args[2][at[0], at[1], 0, 5] = math.inf
+        args[2][at[0], at[1], 1, d - 1] = -math.inf
+    got, want = _run(args, scale).double(), _want(*args, scale)
+    assert not want.isnan().any() and want.isinf().sum() == 2 * news * 8
+    inf = want.isinf()
+    assert torch.equal(got[inf], want[inf])
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11  # as in _check
+    assert ((got - want).abs()[~inf] <= (want.abs() * eps * 1.01 + 2e-6)[~inf]).all()
+
+
+@pytest.mark.parametrize("value", [math.inf, math.nan])
+def test_a_value_that_a_row_does_not_see(value):
+    """At many rows per sequence: an infinity or NaN in V at the last new token
+    reaches the last query only, the rows before it stay finite."""
+    args = _case([500], [40], 8, 2, 128, 16, torch.bfloat16, seed=4)
+    want = _want(*args, 0.1)
+    args[2][args[5][0, 499 // 16], 499 % 16, :, 7] = value
+    got = _run(args, 0.1).double()
+    assert torch.equal(got[39, :, 7].isnan(), torch.full((8,), math.isnan(value)))
+    assert not got[39, :, 7].isfinite().any()
+    assert ((got - want).abs()[:39] <= want.abs()[:39] * 2.0 ** -8 * 1.01 + 2e-6).all()
