@@ -487,26 +487,48 @@ __global__ __launch_bounds__(256) void k_paged_merge(PagedArgs a) {
 // ---------------------------------------------------------------------------
 // P as three parts of the input type that add up to it: fp32 has 24 significand
 // bits, bf16 parts hold 8 each, fp16 parts 11 each. fp16 lacks fp32's exponents,
-// so P enters scaled by 2^14 (kPShift; P <= 2^14 < 65504, and a part below
-// fp16's last step, 2^-24, is 2^-38 of the row's largest P).
+// so P enters scaled by 2^14 (kPShift; P <= 2^14 < 65504). fp16's last step,
+// 2^-24, is 2^-38 of the row's largest P there, too coarse for a small P beside a
+// large V, so the third part is taken 2^24 times its size (kLowScale; at most
+// 2^14, what two parts leave of a P of 2^14 being 2^-10) and summed apart over 32
+// keys: P of 2^-15 of the largest and more is held whole, a smaller one to 2^-51
+// of the largest, below what 65504 P can add to an fp16 output. (Three requests of
+// 500 new tokens on 6,144, 2,500 and 1,111 cached ones, 28 q / 4 kv heads, d = 128:
+// 168 us with the parts summed together, 186 so; bf16 169.)
 template <typename T>
 struct PParts;
 template <>
 struct PParts<BF16> {
-  static constexpr float kPShift = 0.0f;
+  static constexpr float kPShift = 0.0f, kLowScale = 1.0f;
 };
 template <>
 struct PParts<F16> {
-  static constexpr float kPShift = 14.0f;
+  static constexpr float kPShift = 14.0f, kLowScale = 16777216.0f;
 };
 template <typename T>
 __device__ __forceinline__ void part_pair(float x0, float x1, uint32_t (&u)[3]) {
 #pragma unroll
   for (int p = 0; p < 3; ++p) {
+    if (p == 2) {
+      x0 *= PParts<T>::kLowScale;
+      x1 *= PParts<T>::kLowScale;
+    }
     u[p] = pack2<T>(x0, x1);
     x0 -= T::to_f32(static_cast<uint16_t>(u[p]));
     x1 -= T::to_f32(static_cast<uint16_t>(u[p] >> 16));
   }
+}
+
+// V^T operand of a 16-key step: keys r .. r + 3 and r + 8 .. r + 11, dim xx of a
+// key-major tile
+template <typename T, int D>
+__device__ __forceinline__ typename T::vec8 read_vt(const uint16_t* sv16, int r, int xx) {
+  const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (__attribute__((address_space(3))) i16x4*)(sv16 + tile_elem<D>(r, xx)));
+  const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (__attribute__((address_space(3))) i16x4*)(sv16 + tile_elem<D>(r + 8, xx)));
+  const uint2 lo2 = __builtin_bit_cast(uint2, lo), hi2 = __builtin_bit_cast(uint2, hi);
+  return as_vec8<T>(make_uint4(lo2.x, lo2.y, hi2.x, hi2.y));
 }
 
 // One workgroup (4 waves) per (128-row tile of the G query heads of a KV head,
@@ -685,30 +707,55 @@ __global__ __launch_bounds__(256, 2) void k_paged_rows(PagedArgs a) {
         s[t4][v] = __builtin_amdgcn_exp2f(s[t4][v] - ms);
         l_part += s[t4][v];
       }
+      if constexpr (PParts<T>::kLowScale == 1.0f) {
 #pragma unroll
-      for (int hh = 0; hh < 2; ++hh) {
-        uint32_t u[4][3];
+        for (int hh = 0; hh < 2; ++hh) {
+          uint32_t u[4][3];
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          part_pair<T>(s[t4][8 * hh + 2 * e], s[t4][8 * hh + 2 * e + 1], u[e]);
-        typename T::vec8 pb[3];
+          for (int e = 0; e < 4; ++e)
+            part_pair<T>(s[t4][8 * hh + 2 * e], s[t4][8 * hh + 2 * e + 1], u[e]);
+          typename T::vec8 pb[3];
 #pragma unroll
-        for (int p = 0; p < 3; ++p)
-          pb[p] = as_vec8<T>(make_uint4(u[0][p], u[1][p], u[2][p], u[3][p]));
+          for (int p = 0; p < 3; ++p)
+            pb[p] = as_vec8<T>(make_uint4(u[0][p], u[1][p], u[2][p], u[3][p]));
+          const uint16_t* sv16 = reinterpret_cast<const uint16_t*>(sv[buf]);
+          const int r = 32 * t4 + 16 * hh + tr_row;
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt) {
+            const int xx = 32 * dt + tr_col;
+            const typename T::vec8 va = read_vt<T, D>(sv16, r, xx);
+            o[dt] = T::mfma32(va, pb[2], o[dt]);
+            o[dt] = T::mfma32(va, pb[1], o[dt]);
+            o[dt] = T::mfma32(va, pb[0], o[dt]);
+          }
+        }
+      } else {
+        typename T::vec8 pb[2][3];
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh) {
+          uint32_t u[4][3];
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            part_pair<T>(s[t4][8 * hh + 2 * e], s[t4][8 * hh + 2 * e + 1], u[e]);
+#pragma unroll
+          for (int p = 0; p < 3; ++p)
+            pb[hh][p] = as_vec8<T>(make_uint4(u[0][p], u[1][p], u[2][p], u[3][p]));
+        }
         const uint16_t* sv16 = reinterpret_cast<const uint16_t*>(sv[buf]);
-        const int r = 32 * t4 + 16 * hh + tr_row;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
-          const int xx = 32 * dt + tr_col;
-          const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (__attribute__((address_space(3))) i16x4*)(sv16 + tile_elem<D>(r, xx)));
-          const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (__attribute__((address_space(3))) i16x4*)(sv16 + tile_elem<D>(r + 8, xx)));
-          const uint2 lo2 = __builtin_bit_cast(uint2, lo), hi2 = __builtin_bit_cast(uint2, hi);
-          const typename T::vec8 va = as_vec8<T>(make_uint4(lo2.x, lo2.y, hi2.x, hi2.y));
-          o[dt] = T::mfma32(va, pb[2], o[dt]);
-          o[dt] = T::mfma32(va, pb[1], o[dt]);
-          o[dt] = T::mfma32(va, pb[0], o[dt]);
+          f32x16 low = f32x16{};
+#pragma unroll
+          for (int hh = 0; hh < 2; ++hh) {
+            const int r = 32 * t4 + 16 * hh + tr_row, xx = 32 * dt + tr_col;
+            const typename T::vec8 va = read_vt<T, D>(sv16, r, xx);
+            low = T::mfma32(va, pb[hh][2], low);
+            o[dt] = T::mfma32(va, pb[hh][1], o[dt]);
+            o[dt] = T::mfma32(va, pb[hh][0], o[dt]);
+          }
+#pragma unroll
+          for (int v = 0; v < 16; ++v)
+            o[dt][v] = fmaf(low[v], 1.0f / PParts<T>::kLowScale, o[dt][v]);
         }
       }
     }

@@ -204,7 +204,9 @@ int fp_kv_cache_write(const fp_kv_cache_args* a, void* stream);
  * i.e. row t attends to the first used[b] - (cu[b + 1] - 1 - t) cached tokens,
  * and query head h reads KV head h / (num_q_heads / num_kv_heads). Cached token
  * k of sequence b is at page table[b][k / block_size], slot k % block_size.
- * fp32 softmax and sums (the probabilities are not rounded to the input type).
+ * fp32 softmax and sums (the probabilities are not rounded to the input type; a
+ * call of many rows holds one to 2^-51 of its row's largest, in fp16, or to bf16's
+ * smallest step, 2^-133).
  * Replaces vLLM's flash_attn_varlen_func with a block table in the decode
  * branch (patches/patch_loader_vllm_0_12_0.py:201-225,
  * patch_loader_vllm_0_10_0.py:270-368). No host synchronisation: what the host

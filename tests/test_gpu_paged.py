@@ -295,3 +295,29 @@ def test_a_value_that_a_row_does_not_see(value):
     assert torch.equal(got[39, :, 7].isnan(), torch.full((8,), math.isnan(value)))
     assert not got[39, :, 7].isfinite().any()
     assert ((got - want).abs()[:39] <= want.abs()[:39] * 2.0 ** -8 * 1.01 + 2e-6).all()
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("news", [1, 40])
+def test_small_probabilities_of_fp16_calls(d, news):
+    """A value of 60000 at a key of probability 2^-t, 0 at the key that holds the
+    rest: the output is 60000 x 2^-t to half a step of fp16 (2^-25 below its
+    normal range) however far t lies below the row's largest probability."""
+    ts = [12 + i / 8 for i in range(200)]
+    args = _case([64] * len(ts), [news] * len(ts), 4, 1, d, 16, torch.float16, seed=6)
+    q, kc, vc, cu, used, table = args
+    q.zero_()
+    q[..., 0] = 1.0
+    for b, t in enumerate(ts):
+        kc[table[b]] = 0.0
+        kc[table[b], :, :, 0] = -1000.0  # P = 0
+        vc[table[b]] = 0.0
+        kc[table[b, 0], 0, 0, 0] = 0.0
+        kc[table[b, 0], 1, 0, 0] = -t
+        vc[table[b, 0], 1, 0, 3] = 60000.0
+    got, want = _run(args, math.log(2.0)).double(), _want(*args, math.log(2.0))
+    # half a step of the rounded output, and about 2^-20 of the value for the
+    # exponent t <= 37 held in fp32 (2^-19 of a step of one, scale included)
+    step = torch.clamp(2.0 ** (want.abs().clamp_min(1e-30).log2().floor() - 10), min=2.0 ** -24)
+    assert ((got - want).abs() <= 0.5 * step + 2.0 ** -18 * want.abs()).all(), \
+        ((got - want).abs() / step).max()
