@@ -54,19 +54,21 @@ __device__ __forceinline__ int64_t ld_int(const void* p, int is64, int64_t x) {
 }
 
 // One sequence as the workgroups see it. `bad`: more tokens than the block
-// table has room for; its rows are written as NaN.
+// table has room for; its rows are written as NaN. `off`: its query offsets
+// descend or lie outside the call's rows.
 struct PagedSeq {
   int64_t q0;  // first query row
   int nq;      // query rows
   int64_t nk;  // cached tokens
-  bool bad;
+  bool bad, off;
 };
 
 __device__ __forceinline__ PagedSeq paged_seq(const PagedArgs& a, int b) {
   PagedSeq s;
   s.q0 = ld_int(a.cu, a.cu64, b);
   const int64_t q1 = ld_int(a.cu, a.cu64, b + 1);
-  s.nq = s.q0 >= 0 && q1 <= a.T && q1 > s.q0 ? static_cast<int>(q1 - s.q0) : 0;
+  s.off = s.q0 < 0 || q1 > a.T || q1 < s.q0;
+  s.nq = s.off ? 0 : static_cast<int>(q1 - s.q0);
   s.nk = ld_int(a.used, a.used64, b);
   s.bad = s.nk > static_cast<int64_t>(a.width) * a.bs;
   if (s.bad || s.nk < 0) s.nk = 0;
@@ -82,7 +84,9 @@ __device__ __forceinline__ int64_t shfl64(int64_t x, int lane) {
 // The sequence that owns row tile `x` (tiles of `rt` rows of nq * G, numbered
 // over the sequences) and the tile's index in it, or with tok >= 0 the one
 // that owns query row `tok`; and the chunk length all workgroups use. By one
-// wave (64 sequences at a time); b < 0 when there is none.
+// wave (64 sequences at a time); b < 0 when there is none. Where some sequence's
+// offsets do not fit, which rows are whose is unknown: all rows of the call are
+// one sequence's then, and bad.
 struct PagedTile {
   PagedSeq s;
   int b, tl, chunk;
@@ -93,12 +97,14 @@ __device__ __forceinline__ PagedTile paged_find(const PagedArgs& a, int rt, int6
   PagedTile r;
   r.b = -1;
   r.tl = 0;
-  r.s = PagedSeq{0, 0, 0, false};
+  r.s = PagedSeq{0, 0, 0, false, false};
   int64_t carry = 0;
   int maxlen = 0;
+  bool off = false;
   for (int base = 0; base < a.B; base += 64) {
-    PagedSeq s{0, 0, 0, false};
+    PagedSeq s{0, 0, 0, false, false};
     if (base + lane < a.B) s = paged_seq(a, base + lane);
+    off = off || __ballot(s.off) != 0;
     const int tiles =
         static_cast<int>((static_cast<int64_t>(s.nq) * a.G + rt - 1) / rt);
     if (s.nq > 0) maxlen = max(maxlen, static_cast<int>(s.nk));
@@ -126,6 +132,11 @@ __device__ __forceinline__ PagedTile paged_find(const PagedArgs& a, int rt, int6
   for (int o = 1; o < 64; o <<= 1) maxlen = max(maxlen, __shfl_xor(maxlen, o));
   const int per = (maxlen + a.nc - 1) / a.nc;
   r.chunk = (max(per, kPagedMinChunk) + 127) / 128 * 128;
+  if (off) {
+    r.b = tok >= 0 || x < (a.T * a.G + rt - 1) / rt ? 0 : -1;
+    r.tl = static_cast<int>(x);
+    r.s = PagedSeq{0, static_cast<int>(a.T), 0, true, true};
+  }
   // wave-uniform values in scalar registers
   r.b = __builtin_amdgcn_readfirstlane(r.b);
   r.tl = __builtin_amdgcn_readfirstlane(r.tl);

@@ -114,9 +114,11 @@ def paged_decode_attention(query: torch.Tensor, key_cache: torch.Tensor,
     bf16 / fp16 tensors on the GPU (head_dim 64, 128 or 256) take the HIP
     kernels behind ``fp_paged_attention``: no host synchronisation, so what
     only the device sees is checked there (a sequence with more cached tokens
-    than its table row has room for, or a page outside the cache, gets NaN
-    rows). Every other call (CPU, fp32, other head dims or layouts, inputs
-    that require gradients) takes the torch composition."""
+    than its table row has room for, or rows that attend to a page outside the
+    cache, get NaN; offsets that descend or leave the query rows make every
+    row NaN). Every other call (CPU, fp32, other head dims or layouts, offsets
+    or lengths on the host that do not fit, inputs that require gradients)
+    takes the torch composition."""
     if _paged_kernel_takes(query, key_cache, value_cache, out, cu_seqlens_q, seqused_k,
                            block_table):
         _paged_attention_kernel(query, key_cache, value_cache, out, cu_seqlens_q, seqused_k,
@@ -164,6 +166,12 @@ def _paged_kernel_takes(query, key_cache, value_cache, out, cu, used, table) -> 
             used.dtype not in _INDEX or table.dtype not in _INDEX:
         return False
     if table.shape[1] * bs >= 1 << 30 or T * hq >= 1 << 30:
+        return False
+    if not cu.is_cuda:  # known without a synchronisation: refused there
+        at = cu.tolist()
+        if at[0] < 0 or at[-1] > T or any(x > y for x, y in zip(at, at[1:])):
+            return False
+    if not used.is_cuda and any(n > table.shape[1] * bs for n in used[:B].tolist()):
         return False
     return not (torch.is_grad_enabled() and any(t.requires_grad for t in
                                                 (query, key_cache, value_cache, out)))

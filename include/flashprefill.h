@@ -211,9 +211,10 @@ int fp_kv_cache_write(const fp_kv_cache_args* a, void* stream);
  * branch (patches/patch_loader_vllm_0_12_0.py:201-225,
  * patch_loader_vllm_0_10_0.py:270-368). No host synchronisation: what the host
  * cannot see is checked by the kernels. Offsets outside [0, num_tokens] or
- * descending give the sequence no rows; more cached tokens than the table has
- * room for, or a page number outside the cache, make its rows NaN; a row with
- * no cached token to attend to is NaN, a sequence of no cached tokens 0.
+ * descending make every row of the call NaN; more cached tokens than the table
+ * has room for make the sequence's rows NaN, a page number outside the cache the
+ * rows that attend to it; a row with no cached token to attend to is NaN, a
+ * sequence of no cached tokens 0.
  * Strides in elements (multiples of 8, 16-byte aligned bases), head dim
  * contiguous. The integer arrays hold 32- or 64-bit integers. */
 typedef struct fp_paged_args {

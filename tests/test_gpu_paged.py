@@ -321,3 +321,31 @@ def test_small_probabilities_of_fp16_calls(d, news):
     step = torch.clamp(2.0 ** (want.abs().clamp_min(1e-30).log2().floor() - 10), min=2.0 ** -24)
     assert ((got - want).abs() <= 0.5 * step + 2.0 ** -18 * want.abs()).all(), \
         ((got - want).abs() / step).max()
+
+
+@pytest.mark.parametrize("news", [1, 40])
+@pytest.mark.parametrize("hq,hkv,d", [(8, 2, 128), (8, 4, 256)])
+def test_offsets_that_do_not_fit(news, hq, hkv, d):
+    """Query offsets past the tokens, below zero or descending, seen only on the
+    device: every row of the call is NaN. On the host, these and lengths beyond
+    the table are refused."""
+    args = _case([1000, 200, 300], [news] * 3, hq, hkv, d, 16, torch.bfloat16)
+    n = news
+    for cu in ([0, n, 2 * n, 3 * n + 1], [-1, n, 2 * n, 3 * n], [0, 2 * n + 1, 2 * n, 3 * n],
+               [0, n, 2 * n, 2 ** 30]):
+        bad = torch.tensor(cu, dtype=torch.int32)
+        got = _run((*args[:3], bad, *args[4:]), 0.1)
+        assert got.isnan().all(), cu
+        if max(cu) == 2 ** 30:  # (refused only after masks of that size)
+            continue
+        dev = [t.to(DEV) for t in args]
+        with pytest.raises((RuntimeError, IndexError)):
+            vb.paged_decode_attention(*dev[:3], torch.empty_like(dev[0]), bad, *dev[4:], 0.1)
+    dev = [t.to(DEV) for t in args]
+    with pytest.raises(RuntimeError):
+        vb.paged_decode_attention(*dev[:3], torch.empty_like(dev[0]), dev[3],
+                                  args[4] + 16 * args[5].shape[1], dev[5], 0.1)
+    # fewer rows than tokens: the others stay as they were
+    short = torch.tensor([0, n, 2 * n, 3 * n - 1], dtype=torch.int32)
+    got = _run((*args[:3], short, *args[4:]), 0.1)
+    assert (got[3 * n - 1:] == 7.0).all() and not got[:3 * n - 1].isnan().any()
