@@ -139,11 +139,12 @@ def _rows_ok(t: torch.Tensor) -> bool:
 def _paged_kernel_takes(query, key_cache, value_cache, out, cu, used, table) -> bool:
     """Whether the HIP kernels take this call as it is: 16-bit tensors of one
     type on one GPU, head_dim 64 / 128 / 256, 16-byte aligned rows, int32 /
-    int64 metadata of matching shapes, no derivative or functional transform
-    to carry along (dual numbers and vmap see only torch operations)."""
+    int64 metadata of matching shapes, no derivative, functional transform,
+    trace or dispatch mode to carry along (they see only torch operations)."""
     if not query.is_cuda or query.dtype not in _DTYPES:
         return False
-    if forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None:
+    if forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None \
+            or torch._C._get_tracing_state() is not None or torch._C._len_torch_dispatch_stack() > 0:
         return False
     dev, dt = query.device, query.dtype
     if query.dim() != 3 or out.dim() != 3 or key_cache.dim() != 4 or \

@@ -349,3 +349,40 @@ def test_offsets_that_do_not_fit(news, hq, hkv, d):
     short = torch.tensor([0, n, 2 * n, 3 * n - 1], dtype=torch.int32)
     got = _run((*args[:3], short, *args[4:]), 0.1)
     assert (got[3 * n - 1:] == 7.0).all() and not got[:3 * n - 1].isnan().any()
+
+
+def test_transforms_take_the_torch_composition():
+    """vmap, a trace and a dispatch mode see torch operations: a vmapped call is
+    the calls of its slices, and a trace, which cannot follow the lengths, fails
+    instead of recording nothing."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    args = [t.to(DEV) for t in _case([48, 32], [1, 1], 8, 2, 64, 16, torch.bfloat16, spare=0)]
+
+    def call(q):
+        out = torch.zeros_like(q)
+        vb.paged_attention_reference(q, *args[1:3], out, *args[3:], 0.125)
+        return out
+
+    qs = torch.stack([args[0], 2 * args[0], -args[0]])
+    want = torch.stack([call(q) for q in qs])
+
+    def entry(q):
+        out = torch.zeros_like(q)
+        vb.paged_decode_attention(q, *args[1:3], out, *args[3:], 0.125)
+        return out
+
+    # a batched product adds in another order: one rounding to bf16 apart
+    assert torch.allclose(torch.vmap(entry)(qs).float(), want.float(), rtol=2.0 ** -7, atol=1e-5)
+    with pytest.raises(RuntimeError):
+        torch.jit.trace(entry, (qs[0],), check_trace=False)
+
+    class Ops(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, a=(), kw=None):
+            seen.append(func.overloadpacket.__name__)
+            return func(*a, **(kw or {}))
+
+    seen = []
+    with Ops():
+        got = entry(qs[2])
+    assert "copy_" in seen and torch.equal(got, want[2])
