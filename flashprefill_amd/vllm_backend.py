@@ -158,6 +158,10 @@ def _paged_kernel_takes(query, key_cache, value_cache, out, cu, used, table) -> 
     for t in (query, key_cache, value_cache, out):
         if t.dtype != dt or t.device != dev or not _rows_ok(t):
             return False
+    # torch refuses to write these, and so does the composition
+    if any(n > 1 and st == 0 for n, st in zip(out.shape, out.stride())) or \
+            (out.is_inference() and not torch.is_inference_mode_enabled()):
+        return False
     if key_cache.stride(1) >= 1 << 24 or value_cache.stride(1) >= 1 << 24:
         return False
     if cu.dim() != 1 or used.dim() != 1 or table.dim() != 2 or cu.numel() < 2:

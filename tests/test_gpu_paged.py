@@ -386,3 +386,16 @@ def test_transforms_take_the_torch_composition():
     with Ops():
         got = entry(qs[2])
     assert "copy_" in seen and torch.equal(got, want[2])
+
+
+def test_an_output_that_must_not_be_written_is_refused():
+    q, kc, vc, cu, used, table = [t.to(DEV) for t in
+                                  _case([48, 32], [2, 2], 8, 2, 64, 16, torch.bfloat16)]
+    for out in (torch.zeros(1, 8, 64, dtype=q.dtype, device=DEV).expand(4, 8, 64),
+                torch.zeros(4, 1, 64, dtype=q.dtype, device=DEV).expand(4, 8, 64)):
+        with pytest.raises(RuntimeError):
+            vb.paged_decode_attention(q, kc, vc, out, cu, used, table, 0.125)
+    with torch.inference_mode():
+        out = torch.zeros_like(q)
+    with pytest.raises(RuntimeError, match="inference"):
+        vb.paged_decode_attention(q, kc, vc, out, cu, used, table, 0.125)
