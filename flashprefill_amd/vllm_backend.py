@@ -213,6 +213,8 @@ def _paged_attention_kernel(query, key_cache, value_cache, out, cu, used, table,
                          dtype=torch.uint8, device=dev)
         _lib.check(lib.fp_paged_attention(ctypes.byref(a), ws.data_ptr(),
                                           torch.cuda.current_stream(dev).cuda_stream))
+    # a graph that saved `out` finds it changed, as after any in-place operation
+    torch.autograd.graph.increment_version(out)
 
 
 def paged_attention_reference(query: torch.Tensor, key_cache: torch.Tensor,

@@ -399,3 +399,15 @@ def test_an_output_that_must_not_be_written_is_refused():
         out = torch.zeros_like(q)
     with pytest.raises(RuntimeError, match="inference"):
         vb.paged_decode_attention(q, kc, vc, out, cu, used, table, 0.125)
+
+
+def test_the_write_counts_as_an_in_place_change():
+    q, kc, vc, cu, used, table = [t.to(DEV) for t in
+                                  _case([48, 32], [1, 1], 8, 2, 64, 16, torch.bfloat16)]
+    out = torch.ones_like(q)
+    w = torch.ones_like(q, requires_grad=True)
+    y = (w * out).sum()  # saves out
+    with torch.no_grad():
+        vb.paged_decode_attention(q, kc, vc, out, cu, used, table, 0.125)
+    with pytest.raises(RuntimeError, match="inplace"):
+        y.backward()
