@@ -28,9 +28,10 @@
 // workgroups share a CU and one's splitting and softmax runs beside the
 // other's MFMAs), in the swizzled layout of k_attn (conflict free).
 //
-// Values of 2^56 or more, infinities and NaN do not go through the split
-// (x - x1 of an infinity is NaN, and part products could overflow where the
-// value's own product does not): a workgroup that meets one among its queries
+// Values are scaled by 2^24 before the split (kSplitScale: small values keep all
+// their bits). Values of 2^32 or more, infinities and NaN do not go through it
+// (x - x1 of an infinity is NaN, and scaled part products could overflow where
+// the value's own product does not): a workgroup that meets one among its queries
 // or in a tile forms its row (chunk) again with scalar fp32 FMAs at the end.
 //
 // Numerics follow the reference loop: m starts at -inf and l at 1.0, alpha =
@@ -57,12 +58,19 @@
 
 namespace fp {
 
+// Values are split 2^24 times their size: the third part of the smallest fp32
+// value is then a normal bf16 value (unscaled, it runs into bf16's last step,
+// 2^-133, from 2^-110 on down). Scores and O^T come out 2^48 times their size.
+constexpr float kSplitScale = 16777216.0f;
+constexpr float kUnscale = 1.0f / (kSplitScale * kSplitScale);
 // |x| from which a value does not go through the split
-constexpr float kSplitMax = 7.2057594e16f;  // 2^56
+constexpr float kSplitMax = 4294967296.0f;  // 2^32
 
-// x0, x1 -> their three bf16 parts, packed in pairs
+// x0, x1 -> the three bf16 parts of 2^24 times their size, packed in pairs
 __device__ __forceinline__ void split_pair(float x0, float x1, uint32_t& a, uint32_t& b,
                                            uint32_t& c) {
+  x0 *= kSplitScale;
+  x1 *= kSplitScale;
   const uint32_t u0 = __float_as_uint(x0) & 0xffff0000u, u1 = __float_as_uint(x1) & 0xffff0000u;
   a = (u0 >> 16) | u1;
   const float r0 = x0 - __uint_as_float(u0), r1 = x1 - __uint_as_float(u1);
@@ -128,7 +136,7 @@ __global__ __launch_bounds__(2 * BLK, BLK == 128 ? 2 : 1) void k_attn_f32(AttnAr
   const int qrow = 32 * w + l32;
   const int qg = i * BLK + qrow;
   const bool qvalid = qg < L;
-  const float c = a.sm_scale_log2;
+  const float c = a.sm_scale_log2, cs = c * kUnscale;  // cs: of scores from the split
   const float* q = reinterpret_cast<const float*>(a.q);
   const float* kbase = reinterpret_cast<const float*>(a.k) + t0 * a.kst + kvh * a.khs;
   const float* vbase = reinterpret_cast<const float*>(a.v) + t0 * a.vst + kvh * a.vhs;
@@ -283,13 +291,13 @@ __global__ __launch_bounds__(2 * BLK, BLK == 128 ? 2 : 1) void k_attn_f32(AttnAr
           if (key > qrow) s[t4][v] = -INFINITY;
         }
     }
-    // online softmax over this tile (base 2, scores scaled by c)
+    // online softmax over this tile (base 2, scores scaled by cs)
     float smax = -INFINITY;
 #pragma unroll
     for (int t4 = 0; t4 < TT; ++t4)
 #pragma unroll
       for (int v = 0; v < 16; ++v) smax = fmaxf(smax, s[t4][v]);
-    const float m_new = fmaxf(m_run, pair32_max(smax) * c);
+    const float m_new = fmaxf(m_run, pair32_max(smax) * cs);
     // the factor is 1 for every lane once the maximum has settled (NaN, from
     // -inf - -inf, counts as 1 as in the reference)
     if (__ballot(m_new != m_run) != 0) {
@@ -307,7 +315,7 @@ __global__ __launch_bounds__(2 * BLK, BLK == 128 ? 2 : 1) void k_attn_f32(AttnAr
     for (int t4 = 0; t4 < TT; ++t4)
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
-        s[t4][v] = __builtin_amdgcn_exp2f(fmaf(s[t4][v], c, -m_new));
+        s[t4][v] = __builtin_amdgcn_exp2f(fmaf(s[t4][v], cs, -m_new));
         psum += s[t4][v];
       }
     l_part += psum;
@@ -434,6 +442,7 @@ __global__ __launch_bounds__(2 * BLK, BLK == 128 ? 2 : 1) void k_attn_f32(AttnAr
   }
 
   const float l = pair32_sum(l_part);
+  const float unscale = s_big != 0 ? 1.0f : kUnscale;
   if (split) {
     // chunk of a row: unnormalised O^T [BLK][D], then m [BLK], l [BLK]
     float* pp = a.part + (row * a.f32_chunks + chunk) * static_cast<int64_t>(BLK * D + 2 * BLK);
@@ -443,14 +452,15 @@ __global__ __launch_bounds__(2 * BLK, BLK == 128 ? 2 : 1) void k_attn_f32(AttnAr
 #pragma unroll
       for (int g4 = 0; g4 < 4; ++g4)
         *reinterpret_cast<float4*>(orow + 32 * dt + 8 * g4 + 4 * half) =
-            make_float4(o[dt][4 * g4], o[dt][4 * g4 + 1], o[dt][4 * g4 + 2], o[dt][4 * g4 + 3]);
+            make_float4(o[dt][4 * g4] * unscale, o[dt][4 * g4 + 1] * unscale,
+                        o[dt][4 * g4 + 2] * unscale, o[dt][4 * g4 + 3] * unscale);
     if (half == 0) {
       pp[BLK * D + qrow] = m_run;
       pp[BLK * D + BLK + qrow] = l;
     }
     return;
   }
-  const float rcp = 1.0f / l;
+  const float rcp = unscale / l;
   if (qvalid) {
     float* op = reinterpret_cast<float*>(a.o) + (t0 + qg) * a.ost + h * a.ohs;
 #pragma unroll

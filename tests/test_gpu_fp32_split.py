@@ -1,6 +1,6 @@
 """fp32 attention on three-part bf16 products: error against float64 over
 magnitudes, rows in one and in several chunk slots, and the values that do not
-go through the split (2^56 and above, infinities, NaN)."""
+go through the split (2^32 and above, infinities, NaN)."""
 
 import math
 
@@ -50,7 +50,7 @@ def test_error_against_float64(block, d, S, hq, hkv, kscale, vscale):
     assert rel <= 16 * 2.0 ** -24 * (1 + kscale), rel
 
 
-@pytest.mark.parametrize("value", [2.0 ** 56, 1e30, 3.4028234e38, math.inf, -math.inf])
+@pytest.mark.parametrize("value", [2.0 ** 31, 2.0 ** 32, 2.0 ** 56, 1e30, 3.4028234e38, math.inf, -math.inf])
 def test_a_key_of_score_minus_infinity_or_far_below_drops_out(value):
     # keys whose score is hugely negative (or -inf) get P = 0: the rows equal
     # those computed without them, with no NaN from the parts
@@ -107,3 +107,38 @@ def test_sparse_lists_in_chunks_match_one_slot_per_row():
     # the same products; the chunks' merge adds a rounding per chunk
     assert ((o1 - o16[:1]).norm() / o1.norm()).item() <= 8 * 2.0 ** -24
     assert torch.equal(o16[0], o16[15])
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("scale", [1e-32, 1e-34, 1e-35, 1e-36])
+def test_tiny_values_keep_their_bits(d, scale):
+    # V, and K against a Q that makes up for it, near the end of fp32's normal
+    # range (1.2e-38), where the third of three bf16 parts would be a subnormal
+    S = 700
+    g = torch.Generator(device=DEV).manual_seed(d)
+    q = torch.randn(S, 2, d, generator=g, device=DEV)
+    k = torch.randn(S, 1, d, generator=g, device=DEV)
+    # magnitudes above 1 / 16, so that no element is a subnormal of its own
+    v = torch.randn(S, 1, d, generator=g, device=DEV)
+    v = (v + 0.0625 * v.sign()) * scale
+    got, want = _run(q, k, v).double(), _dense(q, k, v)
+    assert ((got - want).norm() / want.norm()).item() <= 32 * 2.0 ** -24
+    up = 2.0 ** 20  # (below the bound of the split)
+    down = scale * 64
+    got, want = _run(q * up, k * down, v / scale).double(), _dense(q * up, k * down, v / scale)
+    assert ((got - want).norm() / want.norm()).item() <= 32 * 2.0 ** -24
+
+
+def test_tiny_probabilities_keep_their_bits():
+    # a V of one non-zero entry at a key of P = 2^-t: the output is P V however
+    # small P is (exp2 of an exponent t held in fp32: 2^-24 t)
+    S, d, H = 128, 64, 64
+    ts = torch.linspace(100, 124, H)
+    q = torch.zeros(S, H, d, device=DEV)
+    k, v = torch.zeros(S, H, d, device=DEV), torch.zeros(S, H, d, device=DEV)
+    q[:, :, 0] = 8 * math.log(2.0)
+    k[1, :, 0] = -ts.to(DEV)
+    k[2:, :, 0] = -1e4  # P = 0
+    v[1, :, 4] = 2.0 ** 20
+    got, want = _run(q, k, v).double()[1:, :, 4], _dense(q, k, v)[1:, :, 4]
+    assert ((got - want) / want).abs().max().item() <= 124 * 4 * 2.0 ** -24
