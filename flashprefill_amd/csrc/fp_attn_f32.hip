@@ -6,11 +6,12 @@
 // or one chunk of a row's list, in the "one query per lane" orientation of
 // k_attn. The fp32 products are formed on the bf16 matrix units, which run 16
 // times as fast as the fp32 ones: every fp32 value is the exact sum of three
-// bf16 parts (8 + 8 + 8 significand bits), x = x1 + x2 + x3 with x1 truncated
-// and x2, x3 rounded to nearest, and
+// bf16 parts (8 + 8 + 8 significand bits), x = x1 + x2 + x3, each rounded to
+// nearest (|x2| <= 2^-8 |x|, |x3| <= 2^-17 |x|), and
 //
 //   x y = x1 y1 + (x1 y2 + x2 y1) + (x1 y3 + x2 y2 + x3 y1) + rest,
-//   |rest| < 2^-22 |x y|, of either sign (about 2^-25 on average),
+//   |rest| <= 2^-24 |x y|, one rounding of an fp32 product, of either sign (about
+//   2^-27 on average; with x1 truncated instead, 2^-22 and 2^-25),
 //
 // i.e. six v_mfma_f32_32x32x16_bf16 (192 cycles) per 16 steps of the sum in
 // place of eight v_mfma_f32_32x32x2_f32 (512 cycles), with fp32 accumulation
@@ -71,9 +72,8 @@ __device__ __forceinline__ void split_pair(float x0, float x1, uint32_t& a, uint
                                            uint32_t& c) {
   x0 *= kSplitScale;
   x1 *= kSplitScale;
-  const uint32_t u0 = __float_as_uint(x0) & 0xffff0000u, u1 = __float_as_uint(x1) & 0xffff0000u;
-  a = (u0 >> 16) | u1;
-  const float r0 = x0 - __uint_as_float(u0), r1 = x1 - __uint_as_float(u1);
+  a = pack2<BF16>(x0, x1);
+  const float r0 = x0 - __uint_as_float(a << 16), r1 = x1 - __uint_as_float(a & 0xffff0000u);
   b = pack2<BF16>(r0, r1);
   c = pack2<BF16>(r0 - __uint_as_float(b << 16), r1 - __uint_as_float(b & 0xffff0000u));
 }

@@ -142,3 +142,40 @@ def test_tiny_probabilities_keep_their_bits():
     v[1, :, 4] = 2.0 ** 20
     got, want = _run(q, k, v).double()[1:, :, 4], _dense(q, k, v)[1:, :, 4]
     assert ((got - want) / want).abs().max().item() <= 124 * 4 * 2.0 ** -24
+
+
+def _small_products(q, k, truncate):
+    """relative weight of the part products that are left out (second by third,
+    third by third), the first parts truncated or rounded to nearest"""
+    def parts(x):
+        x1 = (x.view(torch.int32) & -65536).view(torch.float32) if truncate else x.bfloat16().float()
+        x2 = (x - x1).bfloat16().float()
+        return x2.double(), (x - x1).double() - x2.double()
+    (q2, q3), (k2, k3) = parts(q), parts(k)
+    return ((q2 * k3 + q3 * k2 + q3 * k3) / (q.double() * k.double())).abs()
+
+
+def test_a_score_of_one_product():
+    """Scores that are one product q k each (the other dims are 0), for the pairs
+    whose small part products weigh most: no further off than a rounded product."""
+    g = torch.Generator().manual_seed(11)
+    q = 8 * (1 + torch.rand(1000000, generator=g) / 8)
+    k = -32 * (1 + torch.rand(1000000, generator=g) / 8)
+    top = torch.cat([_small_products(q, k, t).topk(128).indices for t in (False, True)])
+    q, k = q[top], k[top]
+    assert _small_products(q, k, False).max() <= 2.0 ** -24
+    H, d = 256, 64
+    Q = torch.zeros(2, H, d)
+    K, V = torch.zeros(2, H, d), torch.zeros(2, H, d)
+    Q[:, :, 9] = q
+    K[0, :, 9] = k
+    V[0] = 1.0
+    got = _run(Q.to(DEV), K.to(DEV), V.to(DEV)).double().cpu()[1, :, 0]
+    s = (q.double() * k.double()) / 8
+    want = 1 / (1 + torch.exp(-s))
+    # |s| times what its relative error may be: 2^-24 for the product, 2^-24 for its
+    # rounding, 2^-24 for that of the scaled exponent, 2^-26 for the scale's; and
+    # 2^-22 for exp2, the sum and the quotient
+    bound = s.abs() * (3 * 2.0 ** -24 + 2.0 ** -26) + 2.0 ** -22
+    rel = ((got - want) / want).abs()
+    assert (rel <= bound).all(), (rel / bound).max()
