@@ -414,9 +414,14 @@ __global__ __launch_bounds__(2 * BLK, BLK == 128 ? 2 : 1) void k_attn_f32(AttnAr
       for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
         for (int v = 0; v < 16; ++v) o[dt][v] *= alpha;
+      // scores of -inf before the first finite one: P = 0, but NaN (-inf - -inf, as
+      // in the reference, whose tile is the block) where they fill a row's first block
+      const float ms = m_new == -INFINITY ? 0.0f : m_new;
+      if (chunk == 0 && it == BLK / 32 - 1 && m_new == -INFINITY)
+        l_part = __uint_as_float(0x7fc00000u);
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
-        s[v] = __builtin_amdgcn_exp2f(fmaf(s[v], c, -m_new));
+        s[v] = __builtin_amdgcn_exp2f(fmaf(s[v], c, -ms));
         l_part += s[v];
         // the other half-wave holds the P of the key 4 apart
         const float other = __uint_as_float(xchg32(__float_as_uint(s[v])));

@@ -24,10 +24,11 @@ def _dense(q, k, v):
     return torch.matmul(torch.softmax(s, -1), v).permute(1, 0, 2)
 
 
-def _run(q, k, v, block=128):
+def _run(q, k, v, block=128, last_n=2):
     o = torch.empty_like(q)
     cu = torch.tensor([0, q.shape[0]], dtype=torch.int32, device=DEV)
-    flash_prefill_varlen_func(q, k, v, o, cu, q.shape[0], 0.0, block)  # alpha 0: every block
+    # alpha 0: every block (of finite pooled keys; with last_n rows dense, any)
+    flash_prefill_varlen_func(q, k, v, o, cu, q.shape[0], 0.0, block, last_n_block=last_n)
     return o
 
 
@@ -179,3 +180,29 @@ def test_a_score_of_one_product():
     bound = s.abs() * (3 * 2.0 ** -24 + 2.0 ** -26) + 2.0 ** -22
     rel = ((got - want) / want).abs()
     assert (rel <= bound).all(), (rel / bound).max()
+
+
+@pytest.mark.parametrize("d,block", [(64, 128), (128, 128), (128, 64), (64, 64)])
+@pytest.mark.parametrize("hq", [2, 32])
+def test_runs_of_keys_of_score_minus_infinity(d, block, hq):
+    # whole tiles of such keys at the start of a row, of a diagonal block and of a
+    # chunk drop out (2 heads: several chunk slots per row); a row whose first
+    # selected block holds nothing else is NaN, as softmax over that tile is
+    S = 1500
+    g = torch.Generator(device=DEV).manual_seed(d + block)
+    q = torch.rand(S, hq, d, generator=g, device=DEV) + 0.5
+    k = torch.randn(S, 1, d, generator=g, device=DEV)
+    v = torch.randn(S, 1, d, generator=g, device=DEV)
+    gone = torch.zeros(S, dtype=torch.bool, device=DEV)
+    gone[:block - 16] = True
+    gone[2 * block:2 * block + 64] = True
+    gone[4 * block:7 * block] = True
+    kk = k.clone()
+    kk[gone] = -math.inf
+    got = _run(q, kk, v, block, 100).double()
+    want = _dense(q, torch.where(gone[:, None, None], torch.full_like(k, -1e4), k), v)
+    first = block - 16
+    assert got[:first].isnan().all()
+    assert ((got - want)[first:].norm() / want[first:].norm()).item() <= 32 * 2.0 ** -24 * 4
+    kk[:block] = -math.inf
+    assert _run(q, kk, v, block, 100).isnan().all()
