@@ -360,7 +360,10 @@ __device__ __forceinline__ void attn_block_halves(AttnState<T, D>& st, const typ
       for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
         for (int v = 0; v < 16; ++v) st.o[dt][v] *= alpha;
-      ps = exp_pack<T, KP>(s, st.m_run, c, live_p, pk);
+      // A row without a finite score yet: P = 0, and NaN only if the whole block has
+      // none (-inf - -inf, as with the block as one tile)
+      const bool more = p < NP - 1 && (!DIAG || (p + 1) * KP < live);
+      ps = exp_pack<T, KP>(s, more && st.m_run == -INFINITY ? 0.0f : st.m_run, c, live_p, pk);
     }
     st.l_part += ps;
 

@@ -46,3 +46,31 @@ def test_dense_rows(lens, hq, hkv, block, dtype):
         # on every element and a tenth of it on the mean
         bar = 2.0 ** -8 * 5 if dtype == torch.bfloat16 else 2.0 ** -11 * 5
         assert err.max().item() <= bar and err.mean().item() <= bar / 10, (b, n, err.max())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,hq", [(700, 4), (13000, 32)])
+def test_runs_of_keys_of_score_minus_infinity(n, hq, dtype):
+    """A row's first 64-key pass without a finite score drops out, also in a
+    diagonal block; rows that see nothing else in their first block are NaN, as the
+    softmax of that tile is."""
+    d, block, run = 64, 128, 100
+    g = torch.Generator(device=DEV).manual_seed(n)
+    q = (torch.rand(n, hq, d, generator=g, device=DEV) + 0.5).to(dtype)
+    k = torch.randn(n, 1, d, generator=g, device=DEV).to(dtype)
+    v = torch.randn(n, 1, d, generator=g, device=DEV).to(dtype)
+    cu = torch.tensor([0, n], dtype=torch.int32, device=DEV)
+    outs = []
+    for low in (-math.inf, -200.0):  # far below: P = 0 there too
+        kk = k.clone()
+        kk[:run] = low
+        o = torch.empty_like(q)
+        flash_prefill_varlen_func(q, kk, v, o, cu, n, 0.0, block)
+        outs.append(o)
+    assert outs[0][:run].isnan().all()
+    assert not outs[0][run:].isnan().any()
+    # the same scores but for the run's, so P and the sums differ by the maximum
+    # that the first pass leaves: a rounding of P and one of the result
+    err = (outs[0][run:].float() - outs[1][run:].float()).abs()
+    bar = 2.0 ** -8 * 5 if dtype == torch.bfloat16 else 2.0 ** -11 * 5
+    assert err.max().item() <= bar and err.mean().item() <= bar / 10
