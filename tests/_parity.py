@@ -20,6 +20,18 @@ OUT_MAX_ABS_F32 = 1e-4  # fp32 inputs: fp32 MFMA against the oracle's exact-then
 OUT_MEAN_ABS_F32 = 1e-5
 
 
+def persistent_grid_slots(hq: int, lens: Sequence[int], block: int, d: int) -> Tuple[int, int]:
+    """Attention slots of a 16-bit call (one per query head and block of the block
+    table's capacity; split rows add to it) and the least number at which the
+    host launches the persistent grid: four per resident workgroup. A workgroup
+    is block / 32 waves; a SIMD holds one wave at d = 256, three at 64, else two."""
+    nb_max = (max(lens) + block - 1) // block
+    cap = min(len(lens) * nb_max, (sum(lens) + (block - 1) * len(lens)) // block)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    per_cu = {256: 1, 64: 3}.get(d, 2) * 4 // (block // 32)
+    return hq * cap, 4 * ((cus * per_cu + 7) // 8 * 8)
+
+
 def _ulp_line(x: torch.Tensor) -> torch.Tensor:
     """bf16 / fp16 / fp32 bit patterns mapped to a monotone integer line (+0
     and -0 coincide), so that differences count units in the last place."""

@@ -7,7 +7,7 @@ import torch
 from flashprefill_amd import FlashPrefillCall, flash_prefill, flash_prefill_varlen_func
 from flashprefill_amd import _lib
 from oracle import flashprefill_oracle as O
-from tests._parity import OUT_MAX_ABS, OUT_MEAN_ABS
+from tests._parity import OUT_MAX_ABS, OUT_MEAN_ABS, persistent_grid_slots
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -154,14 +154,15 @@ def test_growing_logits_rescale(step):
 @pytest.mark.parametrize("block,dtype,d", [(128, torch.bfloat16, 128), (64, torch.bfloat16, 128),
                                            (128, torch.float16, 64)])
 def test_persistent_attention_queues_rearm(block, dtype, d):
-    # 16K (block 128) / 32K (block 64) tokens x 32 heads give at least 8
-    # attention slots per resident workgroup, so the attention stage runs as
-    # the persistent grid over per-XCD claim queues. The plan kernel empties
+    # 16K (block 128) / 32K (block 64) tokens x 32 heads: the attention stage
+    # runs as the persistent grid over per-XCD claim queues. The plan kernel empties
     # the queues once; every attention launch after that must empty them
     # again itself: attention-only launches repeated on the planned
     # workspace, and a second full call, give the first call's output bit for
     # bit.
     T, Hq, Hkv = 16384 if block == 128 else 32768, 32, 8
+    slots, least = persistent_grid_slots(Hq, [T], block, d)
+    assert slots >= least
     q, k, v = (_rand((T, Hq, d), 41, dtype, scale=1.5).to(DEV),
                _rand((T, Hkv, d), 42, dtype, scale=1.5).to(DEV), _rand((T, Hkv, d), 43, dtype).to(DEV))
     cu = torch.tensor([0, T], dtype=torch.int32, device=DEV)

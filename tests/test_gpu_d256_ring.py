@@ -9,6 +9,7 @@ import pytest
 import torch
 
 from flashprefill_amd import flash_prefill_varlen_func
+from tests._parity import persistent_grid_slots
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -52,6 +53,9 @@ def test_rows_of_few_blocks(lens, block, dtype):
     _check(lens, 4, 2, block, dtype)
 
 
-@pytest.mark.parametrize("block,lens", [(128, [2100, 1900]), (64, [1500, 1700])])
-def test_persistent_grid_and_split_rows(block, lens):
-    _check(lens, 32, 8, block, torch.bfloat16)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("block,lens", [(128, [2100, 1900]), (64, [2300, 2500])])
+def test_persistent_grid_and_split_rows(block, lens, dtype):
+    slots, least = persistent_grid_slots(32, lens, block, 256)
+    assert slots >= least
+    _check(lens, 32, 8, block, dtype)

@@ -9,6 +9,7 @@ import pytest
 import torch
 
 from flashprefill_amd import flash_prefill_varlen_func
+from tests._parity import persistent_grid_slots
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -19,8 +20,11 @@ DEV = "cuda:0"
 @pytest.mark.parametrize("lens,hq,hkv", [([1, 31, 32, 33, 63, 64, 65], 4, 2),
                                          ([96, 127, 128, 129, 191, 192, 193], 4, 1),
                                          ([255, 256, 257, 320, 0, 385], 6, 3),
-                                         ([3000, 2900], 32, 8)])
+                                         ([6300, 6200], 32, 8)])
 def test_dense_rows(lens, hq, hkv, block, dtype):
+    if hq == 32:
+        slots, least = persistent_grid_slots(hq, lens, block, 64)
+        assert slots >= least
     g = torch.Generator(device=DEV).manual_seed(sum(lens) + block)
     T, d = sum(lens), 64
     q = torch.randn(T, hq, d, generator=g, device=DEV).to(dtype)
@@ -55,6 +59,8 @@ def test_runs_of_keys_of_score_minus_infinity(n, hq, dtype):
     diagonal block; rows that see nothing else in their first block are NaN, as the
     softmax of that tile is."""
     d, block, run = 64, 128, 100
+    slots, least = persistent_grid_slots(hq, [n], block, d)
+    assert (slots >= least) == (hq == 32)
     g = torch.Generator(device=DEV).manual_seed(n)
     q = (torch.rand(n, hq, d, generator=g, device=DEV) + 0.5).to(dtype)
     k = torch.randn(n, 1, d, generator=g, device=DEV).to(dtype)

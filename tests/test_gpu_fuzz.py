@@ -20,7 +20,7 @@ import torch
 
 from flashprefill_amd import synth
 from tests._parity import (OUT_MAX_ABS, OUT_MAX_ABS_F32, OUT_MEAN_ABS, OUT_MEAN_ABS_F32,
-                           assert_pool, run_stages)
+                           assert_pool, persistent_grid_slots, run_stages)
 
 pytestmark = pytest.mark.gpu
 
@@ -143,8 +143,8 @@ def test_random_configuration_wide_blocks_and_head_dims(seed):
 
 
 def _large_case(seed):
-    """Ragged batches large enough that the attention stage runs as the
-    persistent grid (at least 8 work slots per resident workgroup)."""
+    """Ragged batches; the test grows them until the attention stage runs as the
+    persistent grid."""
     rnd = random.Random(seed)
     block = rnd.choice([64, 128])
     hkv = rnd.choice([2, 4, 8])
@@ -162,15 +162,11 @@ def _large_case(seed):
 @pytest.mark.parametrize("seed", range(4))
 def test_random_large_configuration_persistent_attention(seed):
     lens, hq, hkv, d, dtype, params, block = _large_case(2000 + seed)
-    per_cu = 2 if block == 128 else 4
-    cus = torch.cuda.get_device_properties(0).multi_processor_count
-    # grow the longest sequence until Hq * (capacity of the block table) reaches
-    # 8 slots per resident workgroup, twice the host's threshold (4) for the
-    # persistent grid, so that every workgroup claims several slots
+    # grow the longest sequence until the slots reach twice the host's threshold
+    # for the persistent grid, so that every workgroup claims several
     while True:
-        nb_max = (max(lens) + block - 1) // block
-        cap = min(len(lens) * nb_max, (sum(lens) + (block - 1) * len(lens)) // block)
-        if hq * cap >= 8 * per_cu * cus:
+        slots, least = persistent_grid_slots(hq, lens, block, d)
+        if slots >= 2 * least:
             break
         lens[lens.index(max(lens))] += 4096
     # the structured synthetic distribution of the benchmark (sinks, stripes,
