@@ -256,8 +256,9 @@ __device__ __forceinline__ void attn_block(AttnState<T, D>& st, const typename T
 // S, the V refill the last pass's P.V; the V wait precedes the first pass's P.V.
 // (This is the online softmax over 64-key tiles, a K_TILE_SIZE the reference
 // runs.) Measured against the whole block at once and two waves per SIMD (one
-// MI355X, 32 q / 8 kv heads, attention alone): 32K 711 -> 689 us, 8K 137 -> 131,
-// 16K with every block 1,089 -> 1,059 (1,046 TFLOP/s). Blocks of 64 keys need 148
+// MI355X, 32 q / 8 kv heads, whole calls): 32K bf16 999 -> 950 us, 4 x 8K fp16 with
+// a budget 769 -> 747, 4K bf16 93.6 -> 94.3 (few rows per SIMD there; attention alone
+// with every block of 16K 1,089 -> 1,059, 1,046 TFLOP/s). Blocks of 64 keys need 148
 // registers as they are: three waves there too, 16K 246 -> 214 us.
 template <typename T, int D, int BLK, bool DIAG>
 __device__ __forceinline__ void attn_block_halves(AttnState<T, D>& st, const typename T::vec8* qb,
@@ -337,13 +338,19 @@ __device__ __forceinline__ void attn_block_halves(AttnState<T, D>& st, const typ
         }
       }
     }
-    // conditional rescaling as in attn_block, per pass
+    // Conditional rescaling as in attn_block, per pass: always in a row's first block,
+    // so that the block leaves its own maximum as one tile would, then from a quarter
+    // of the sum on, since half the keys reach kRescaleSum later (a row's largest P is
+    // exact where it is the maximum's, 1, and rounded else): 2-norm error against
+    // float64, 6,081 structured tokens, bf16: 2.015e-3 as one tile, 2.021e-3 with
+    // kRescaleSum per pass, 2.000e-3 so (32K bf16 call 933 -> 950 us, 4 x 8K fp16 743
+    // -> 747, 4K unchanged).
     uint32_t pk[KP][8];
     float ps = 0.0f;
     bool move = first && p == 0;
     if (!move) {
       ps = exp_pack<T, KP>(s, st.m_run, c, live_p, pk);
-      move = __ballot(!(ps <= kRescaleSum)) != 0;
+      move = first || __ballot(!(ps <= 0.25f * kRescaleSum)) != 0;
     }
     if (move) {
       float mx = -INFINITY;
