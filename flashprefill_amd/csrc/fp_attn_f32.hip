@@ -17,7 +17,7 @@
 // place of eight v_mfma_f32_32x32x2_f32 (512 cycles), with fp32 accumulation
 // and fewer roundings of the running sum (6 instead of 8 per 16 terms). Against
 // float64 the outputs are no further off than with the fp32 units (2-norm error
-// 1.1e-6, there 1.5e-6, on structured 4K inputs).
+// 1.2e-6, there 1.7e-6, on structured 4K inputs).
 //
 //   S^T = K . Q^T    A = K parts from LDS, B = Q^T parts in registers
 //   O^T += V^T . P^T A = V^T parts via ds_read_b64_tr_b16 from the key-major
@@ -50,11 +50,12 @@
 //
 // Measured (one MI355X), attention alone, against the fp32 units with tiles
 // staged between two barriers and one workgroup per row: 4K x 8 q / 2 kv heads,
-// d = 64: 324 -> 98 us; the same at d = 128: 636 -> 218; 4K x 32 q / 8 kv heads,
-// d = 128: 876 -> 515 us (149 TFLOP/s; the fp32 units' peak is 157); 8K x 32
-// heads, d = 64: 1,125 -> 610 us. The bf16 units are ~40 % busy there: the
-// splitting, softmax and conversion instructions of a tile (~650) take about as
-// long as its 96 MFMAs and two waves per SIMD overlap them only in part.
+// d = 64: 315 -> 94 us; the same at d = 128: 630 -> 202; 4K x 32 q / 8 kv heads,
+// d = 128: 824 -> 465 us; 8K x 32 heads, d = 64: 1,068 -> 526 us. (Scaling and
+// rounding the first parts cost 2 - 4 % of it.) The bf16 units are ~40 % busy
+// there: the scaling, splitting, softmax and conversion instructions of a tile
+// (~700) take about as long as its 96 MFMAs and two waves per SIMD overlap them
+// only in part.
 #include "fp_attn_common.h"
 
 namespace fp {

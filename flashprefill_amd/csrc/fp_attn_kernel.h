@@ -258,7 +258,7 @@ __device__ __forceinline__ void attn_block(AttnState<T, D>& st, const typename T
 // runs.) Measured against the whole block at once and two waves per SIMD (one
 // MI355X, 32 q / 8 kv heads, whole calls): 32K bf16 999 -> 950 us, 4 x 8K fp16 with
 // a budget 769 -> 747, 4K bf16 93.6 -> 94.3 (few rows per SIMD there; attention alone
-// with every block of 16K 1,089 -> 1,059, 1,046 TFLOP/s). Blocks of 64 keys need 148
+// with every block of 16K 1,135 -> 1,115, 993 TFLOP/s). Blocks of 64 keys need 147
 // registers as they are: three waves there too, 16K 246 -> 214 us.
 template <typename T, int D, int BLK, bool DIAG>
 __device__ __forceinline__ void attn_block_halves(AttnState<T, D>& st, const typename T::vec8* qb,

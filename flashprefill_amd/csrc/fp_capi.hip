@@ -178,8 +178,9 @@ int layout(const fp_problem* p, fp_ws_layout* L) {
   // C is about one workgroup slot's share of the attention, estimated from
   // below before the selection exists: every row's forced blocks (sink,
   // window and min_budget; at least the diagonal) plus the last_n rows' full
-  // lists, over the resident slots of an MI355X (256 CUs; the count only sets
-  // the balance). A chunk longer than a slot's share becomes the kernel's
+  // lists, over the resident slots of an MI355X (256 CUs; two workgroups each at
+  // d = 64 as well, where three are resident: the count only sets the balance). A
+  // chunk longer than a slot's share becomes the kernel's
   // critical path (one TP = 8 shard of a 128K sequence, 4 q / 1 kv heads:
   // attention 0.80 ms with 256-block chunks, 0.74 ms with 64); a much shorter
   // one adds per-chunk work (first loads, partial store, merge; 16-block
@@ -569,7 +570,10 @@ int paged_valid(const fp_paged_args* a) {
 // us with 512, 176 with 1024, 205 with 2048.) The line between the kernels: 8
 // sequences of 3,000 tokens, 32 q / 8 kv heads, with 4, 8, 16 and 64 queries each
 // (16, 32, 64 and 256 rows): k_paged 147 (32 of 4,000), 49, 84 and 254 us,
-// k_paged_rows 153, 46, 45 and 90.
+// k_paged_rows 153, 46, 45 and 90. The average decides, since only the device sees
+// the sequences: one of 4,000 tokens with 2,000 new ones beside 60 of 8,000 with one
+// query each runs in k_paged_rows as a whole, one chunk per row, 690 - 725 us, where
+// the two kinds as calls of their own take 245 - 250 and 395.
 struct PagedSplit {
   bool many;  // k_paged_rows
   int64_t tiles;

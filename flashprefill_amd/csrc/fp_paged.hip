@@ -34,9 +34,10 @@
 //
 // Measured (one MI355X, d = 128): 32 sequences of 300 .. 15,300 tokens (32 q /
 // 8 kv heads, 0.9 GB of cache) 18.8 ms per call as per-sequence torch gathers
-// and fp32 products, 0.22 ms here (k_paged 0.21 ms = 4.2 TB/s, where a 2 GiB
-// copy reaches 5.0; k_paged_merge 6 us); one sequence of 65,000 tokens 6.57 ->
-// 0.058 ms (127 chunks x 8 KV heads; k_paged 49 us = 5.4 TB/s).
+// and fp32 products, 0.22 ms here (k_paged 0.20 - 0.21 ms = 4.2 - 4.5 TB/s, where
+// a 1 GiB copy reaches 5.24; k_paged_merge 6 us); one sequence of 65,000 tokens
+// 6.57 -> 0.056 ms a call among others of its kind, 0.066 with inputs that change
+// (127 chunks x 8 KV heads; k_paged 49 us = 5.4 TB/s, k_paged_merge 7).
 #include "fp_attn_common.h"
 
 namespace fp {
@@ -550,9 +551,10 @@ __device__ __forceinline__ typename T::vec8 read_vt(const uint16_t* sv16, int r,
 // share every K / V byte, where k_paged reads them once per 16 rows. P stays
 // fp32: P.V runs on its three exact 16-bit parts (48 of the 64 MFMAs of a tile
 // and wave at d = 128). Bound by these MFMAs and the instructions that form the
-// parts. Measured (one MI355X): 500 new tokens each on 6,144, 2,500 and 1,111
-// cached ones (28 q / 4 kv heads, d = 128) 504 us with k_paged, 172 here; 4 x
-// 2,048 new of 4,096 (32 q / 8 kv) 3,045 -> 890 us = 463 TFLOP/s (924 of MFMAs).
+// parts. Measured (one MI355X, whole calls): 500 new tokens each on 6,144, 2,500
+// and 1,111 cached ones (28 q / 4 kv heads, d = 128) 504 us with k_paged, 169 here
+// (the merge 8); 4 x 2,048 new of 4,096 (32 q / 8 kv) 3,045 -> 890 us = 463 TFLOP/s
+// (924 of MFMAs).
 template <typename T, int D, bool P16>
 __global__ __launch_bounds__(256, 2) void k_paged_rows(PagedArgs a) {
   constexpr int KT = 64, TT = KT / 32;

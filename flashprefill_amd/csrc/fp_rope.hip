@@ -24,7 +24,8 @@
 // t minus the start of the last sequence that begins at or before t. The offsets
 // of a batch (at most kRopeMaxBatch) sit in LDS. (As torch steps, the positions
 // of a packed batch were seven launches per layer: a layer of 16384 tokens took
-// 2107 us with them, 2091 with the offsets. The kernel itself takes 76 - 80 us for
+// 2103 us with them and 2083 with the offsets on one box, the same within the spread
+// of the runs on others. The kernel itself takes 76 - 80 us for
 // 36 heads of 128 there, 302 MB at 4 TB/s; 32-bit row arithmetic in place of the
 // 64-bit division did not change that.)
 #include "fp_internal.h"
