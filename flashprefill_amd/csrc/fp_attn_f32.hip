@@ -29,10 +29,9 @@
 // workgroups share a CU and one's splitting and softmax runs beside the
 // other's MFMAs), in the swizzled layout of k_attn (conflict free).
 //
-// Values are scaled by 2^24 before the split (kSplitScale: small values keep all
-// their bits). Values of 2^32 or more, infinities and NaN do not go through it
-// (x - x1 of an infinity is NaN, and scaled part products could overflow where
-// the value's own product does not): a workgroup that meets one among its queries
+// Values of 2^56 or more, infinities and NaN do not go through the split
+// (x - x1 of an infinity is NaN, and part products could overflow where the
+// value's own product does not): a workgroup that meets one among its queries
 // or in a tile forms its row (chunk) again with scalar fp32 FMAs at the end.
 //
 // Numerics follow the reference loop: m starts at -inf and l at 1.0, alpha =
@@ -51,8 +50,8 @@
 // Measured (one MI355X), attention alone, against the fp32 units with tiles
 // staged between two barriers and one workgroup per row: 4K x 8 q / 2 kv heads,
 // d = 64: 315 -> 94 us; the same at d = 128: 630 -> 202; 4K x 32 q / 8 kv heads,
-// d = 128: 824 -> 465 us; 8K x 32 heads, d = 64: 1,068 -> 526 us. (Scaling and
-// rounding the first parts cost 2 - 4 % of it.) The bf16 units are ~40 % busy
+// d = 128: 824 -> 465 us; 8K x 32 heads, d = 64: 1,068 -> 526 us. (Scaling V and P and
+// rounding the first parts cost 1 - 3 % of it.) The bf16 units are ~40 % busy
 // there: the scaling, splitting, softmax and conversion instructions of a tile
 // (~700) take about as long as its 96 MFMAs and two waves per SIMD overlap them
 // only in part.
@@ -60,19 +59,21 @@
 
 namespace fp {
 
-// Values are split 2^24 times their size: the third part of the smallest fp32
+// P and V are split 2^24 times their size: the third part of the smallest fp32
 // value is then a normal bf16 value (unscaled, it runs into bf16's last step,
-// 2^-133, from 2^-110 on down). Scores and O^T come out 2^48 times their size.
+// 2^-133, from 2^-110 on down), and O^T comes out 2^48 times its size. Q and K are
+// split as they are: a K below 2^-110 has scores below 2^-47 beside any Q that goes
+// through the split, which exp2 does not see.
 constexpr float kSplitScale = 16777216.0f;
 constexpr float kUnscale = 1.0f / (kSplitScale * kSplitScale);
 // |x| from which a value does not go through the split
-constexpr float kSplitMax = 4294967296.0f;  // 2^32
+constexpr float kSplitMax = 7.2057594e16f;  // 2^56
 
-// x0, x1 -> the three bf16 parts of 2^24 times their size, packed in pairs
-__device__ __forceinline__ void split_pair(float x0, float x1, uint32_t& a, uint32_t& b,
-                                           uint32_t& c) {
-  x0 *= kSplitScale;
-  x1 *= kSplitScale;
+// x0, x1 (times `scale`) -> their three bf16 parts, packed in pairs
+__device__ __forceinline__ void split_pair(float x0, float x1, float scale, uint32_t& a,
+                                           uint32_t& b, uint32_t& c) {
+  x0 *= scale;
+  x1 *= scale;
   a = pack2<BF16>(x0, x1);
   const float r0 = x0 - __uint_as_float(a << 16), r1 = x1 - __uint_as_float(a & 0xffff0000u);
   b = pack2<BF16>(r0, r1);
@@ -137,7 +138,7 @@ __global__ __launch_bounds__(2 * BLK, BLK == 128 ? 2 : 1) void k_attn_f32(AttnAr
   const int qrow = 32 * w + l32;
   const int qg = i * BLK + qrow;
   const bool qvalid = qg < L;
-  const float c = a.sm_scale_log2, cs = c * kUnscale;  // cs: of scores from the split
+  const float c = a.sm_scale_log2;
   const float* q = reinterpret_cast<const float*>(a.q);
   const float* kbase = reinterpret_cast<const float*>(a.k) + t0 * a.kst + kvh * a.khs;
   const float* vbase = reinterpret_cast<const float*>(a.v) + t0 * a.vst + kvh * a.vhs;
@@ -179,7 +180,7 @@ __global__ __launch_bounds__(2 * BLK, BLK == 128 ? 2 : 1) void k_attn_f32(AttnAr
   auto big4 = [](float m, const float4& x) {
     return fmaxf(fmaxf(fmaxf(m, fabsf(x.x)), fmaxf(fabsf(x.y), fabsf(x.z))), fabsf(x.w));
   };
-  auto store_split = [&](uint4 (&dst)[3][KT * CH], const float4 (&x)[PC][2]) {
+  auto store_split = [&](uint4 (&dst)[3][KT * CH], const float4 (&x)[PC][2], float scale) {
 #pragma unroll
     for (int p = 0; p < PC; ++p) {
       const int cidx = t + p * NT;
@@ -187,8 +188,9 @@ __global__ __launch_bounds__(2 * BLK, BLK == 128 ? 2 : 1) void k_attn_f32(AttnAr
       uint32_t u[3][4];
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
-        split_pair(x[p][e].x, x[p][e].y, u[0][2 * e], u[1][2 * e], u[2][2 * e]);
-        split_pair(x[p][e].z, x[p][e].w, u[0][2 * e + 1], u[1][2 * e + 1], u[2][2 * e + 1]);
+        split_pair(x[p][e].x, x[p][e].y, scale, u[0][2 * e], u[1][2 * e], u[2][2 * e]);
+        split_pair(x[p][e].z, x[p][e].w, scale, u[0][2 * e + 1], u[1][2 * e + 1],
+                   u[2][2 * e + 1]);
       }
       const int at = r * CH + ((cidx % CH) ^ swz<D>(r));
 #pragma unroll
@@ -213,8 +215,8 @@ __global__ __launch_bounds__(2 * BLK, BLK == 128 ? 2 : 1) void k_attn_f32(AttnAr
     uint32_t u[3][4];
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
-      split_pair(x[e].x, x[e].y, u[0][2 * e], u[1][2 * e], u[2][2 * e]);
-      split_pair(x[e].z, x[e].w, u[0][2 * e + 1], u[1][2 * e + 1], u[2][2 * e + 1]);
+      split_pair(x[e].x, x[e].y, 1.0f, u[0][2 * e], u[1][2 * e], u[2][2 * e]);
+      split_pair(x[e].z, x[e].w, 1.0f, u[0][2 * e + 1], u[1][2 * e + 1], u[2][2 * e + 1]);
     }
 #pragma unroll
     for (int p = 0; p < 3; ++p)
@@ -239,8 +241,8 @@ __global__ __launch_bounds__(2 * BLK, BLK == 128 ? 2 : 1) void k_attn_f32(AttnAr
 #pragma unroll
     for (int p = 0; p < PC; ++p)
       mx = big4(big4(big4(big4(mx, kf[p][0]), kf[p][1]), vf[p][0]), vf[p][1]);
-    store_split(sk, kf);
-    store_split(sv, vf);
+    store_split(sk, kf, 1.0f);
+    store_split(sv, vf, kSplitScale);
     if (mx >= kSplitMax) s_big = 1;  // (a NaN alone goes through the split as it is)
     if (it + 1 < ntiles) load_tile(it + 1);  // flies during this tile's products
     // the LDS stores are done; the register loads may still be in flight
@@ -292,13 +294,13 @@ __global__ __launch_bounds__(2 * BLK, BLK == 128 ? 2 : 1) void k_attn_f32(AttnAr
           if (key > qrow) s[t4][v] = -INFINITY;
         }
     }
-    // online softmax over this tile (base 2, scores scaled by cs)
+    // online softmax over this tile (base 2, scores scaled by c)
     float smax = -INFINITY;
 #pragma unroll
     for (int t4 = 0; t4 < TT; ++t4)
 #pragma unroll
       for (int v = 0; v < 16; ++v) smax = fmaxf(smax, s[t4][v]);
-    const float m_new = fmaxf(m_run, pair32_max(smax) * cs);
+    const float m_new = fmaxf(m_run, pair32_max(smax) * c);
     // the factor is 1 for every lane once the maximum has settled (NaN, from
     // -inf - -inf, counts as 1 as in the reference)
     if (__ballot(m_new != m_run) != 0) {
@@ -316,7 +318,7 @@ __global__ __launch_bounds__(2 * BLK, BLK == 128 ? 2 : 1) void k_attn_f32(AttnAr
     for (int t4 = 0; t4 < TT; ++t4)
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
-        s[t4][v] = __builtin_amdgcn_exp2f(fmaf(s[t4][v], cs, -m_new));
+        s[t4][v] = __builtin_amdgcn_exp2f(fmaf(s[t4][v], c, -m_new));
         psum += s[t4][v];
       }
     l_part += psum;
@@ -331,7 +333,8 @@ __global__ __launch_bounds__(2 * BLK, BLK == 128 ? 2 : 1) void k_attn_f32(AttnAr
         uint32_t u[3][4];
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          split_pair(s[t4][8 * hh + 2 * e], s[t4][8 * hh + 2 * e + 1], u[0][e], u[1][e], u[2][e]);
+          split_pair(s[t4][8 * hh + 2 * e], s[t4][8 * hh + 2 * e + 1], kSplitScale, u[0][e],
+                     u[1][e], u[2][e]);
         bf16x8 pb[3];
 #pragma unroll
         for (int p = 0; p < 3; ++p)

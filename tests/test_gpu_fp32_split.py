@@ -1,6 +1,6 @@
 """fp32 attention on three-part bf16 products: error against float64 over
 magnitudes, rows in one and in several chunk slots, and the values that do not
-go through the split (2^32 and above, infinities, NaN)."""
+go through the split (2^56 and above, infinities, NaN)."""
 
 import math
 
@@ -119,6 +119,10 @@ def test_tiny_values_keep_their_bits(d, scale):
     g = torch.Generator(device=DEV).manual_seed(d)
     q = torch.randn(S, 2, d, generator=g, device=DEV)
     k = torch.randn(S, 1, d, generator=g, device=DEV)
+    if scale == 1e-32:  # and near the split's upper end, 2^56 = 7.2e16
+        v = torch.randn(S, 1, d, generator=g, device=DEV).clamp(-7, 7) * 1e16
+        got, want = _run(q * 1e-16, k * 1e16, v).double(), _dense(q * 1e-16, k * 1e16, v)
+        assert ((got - want).norm() / want.norm()).item() <= 32 * 2.0 ** -24
     # magnitudes above 1 / 16, so that no element is a subnormal of its own
     v = torch.randn(S, 1, d, generator=g, device=DEV)
     v = (v + 0.0625 * v.sign()) * scale
