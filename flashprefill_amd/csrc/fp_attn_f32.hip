@@ -382,18 +382,16 @@ __global__ __launch_bounds__(2 * BLK, BLK == 128 ? 2 : 1) void k_attn_f32(AttnAr
 
   // Values that the split does not take: the row again, with scalar products
   // (32 keys at a time; accumulator element v of a tile is key 8 (v / 4) +
-  // 4 half + v % 4, o[dt][x] is dim 32 dt + 8 (x / 4) + 4 half + x % 4).
+  // 4 half + v % 4, o[dt][x] is dim 32 dt + 8 (x / 4) + 4 half + x % 4). The
+  // maximum of the whole row comes first, also for a chunk of it, so that no sum of
+  // P V is larger on the way than in the result.
   __syncthreads();
   if (s_big != 0) {
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) o[dt] = f32x16{};
-    m_run = -INFINITY;
-    l_part = half == 0 && !split ? 1.0f : 0.0f;
-#pragma unroll 1
-    for (int it = 0; it < ncnt * (BLK / 32); ++it) {
-      const int j = min(max(sld(list + it / (BLK / 32)), 0), i);
+    // scores of tile `it` of the walk over `blocks`
+    auto scores = [&](const int32_t* blocks, int it, f32x16& s) {
+      const int j = min(max(sld(blocks + it / (BLK / 32)), 0), i);
       const int key0 = 32 * (it % (BLK / 32));
-      f32x16 s = f32x16{};
+      s = f32x16{};
 #pragma unroll 1
       for (int d = 0; d < D; ++d) {
         const float qd = qvalid ? qptr[d] : 0.0f;
@@ -403,26 +401,33 @@ __global__ __launch_bounds__(2 * BLK, BLK == 128 ? 2 : 1) void k_attn_f32(AttnAr
           s[v] = fmaf(qd, kbase[static_cast<int64_t>(min(j * BLK + key, L - 1)) * a.kst + d], s[v]);
         }
       }
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        if (j == i && key0 + 8 * (v >> 2) + 4 * half + (v & 3) > qrow) s[v] = -INFINITY;
+    };
+    m_run = -INFINITY;
+    l_part = 0.0f;
+#pragma unroll 1
+    for (int it = 0; it < nsel * (BLK / 32); ++it) {
+      f32x16 s;
+      scores(a.idx + row_tri, it, s);
       float smax = -INFINITY;
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        if (j == i && key0 + 8 * (v >> 2) + 4 * half + (v & 3) > qrow) s[v] = -INFINITY;
-        smax = fmaxf(smax, s[v]);
-      }
-      const float m_new = fmaxf(m_run, pair32_max(smax) * c);
-      float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-      if (alpha != alpha) alpha = 1.0f;
-      m_run = m_new;
-      l_part *= alpha;
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) o[dt][v] *= alpha;
-      // scores of -inf before the first finite one: P = 0, but NaN (-inf - -inf, as
-      // in the reference, whose tile is the block) where they fill a row's first block
-      const float ms = m_new == -INFINITY ? 0.0f : m_new;
-      if (chunk == 0 && it == BLK / 32 - 1 && m_new == -INFINITY)
+      for (int v = 0; v < 16; ++v) smax = fmaxf(smax, s[v]);
+      m_run = fmaxf(m_run, pair32_max(smax) * c);
+      // scores of -inf are P = 0, but NaN (-inf - -inf, as in the reference, whose
+      // tile is the block) where they fill a row's first block
+      if (chunk == 0 && it == BLK / 32 - 1 && m_run == -INFINITY)
         l_part = __uint_as_float(0x7fc00000u);
+    }
+    const float ms = m_run == -INFINITY ? 0.0f : m_run;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) o[dt] = f32x16{};
+#pragma unroll 1
+    for (int it = 0; it < ncnt * (BLK / 32); ++it) {
+      const int key0 = min(max(sld(list + it / (BLK / 32)), 0), i) * BLK + 32 * (it % (BLK / 32));
+      f32x16 s;
+      scores(list, it, s);
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         s[v] = __builtin_amdgcn_exp2f(fmaf(s[v], c, -ms));
@@ -433,8 +438,7 @@ __global__ __launch_bounds__(2 * BLK, BLK == 128 ? 2 : 1) void k_attn_f32(AttnAr
         for (int hh = 0; hh < 2; ++hh) {
           const int key = key0 + 8 * (v >> 2) + 4 * hh + (v & 3);
           const float p = hh == half ? s[v] : other;
-          const float* vp =
-              vbase + static_cast<int64_t>(min(j * BLK + key, L - 1)) * a.vst + 4 * half;
+          const float* vp = vbase + static_cast<int64_t>(min(key, L - 1)) * a.vst + 4 * half;
 #pragma unroll
           for (int dt = 0; dt < DT; ++dt)
 #pragma unroll

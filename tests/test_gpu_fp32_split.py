@@ -210,3 +210,22 @@ def test_runs_of_keys_of_score_minus_infinity(d, block, hq):
     assert ((got - want)[first:].norm() / want[first:].norm()).item() <= 32 * 2.0 ** -24 * 4
     kk[:block] = -math.inf
     assert _run(q, kk, v, block, 100).isnan().all()
+
+
+@pytest.mark.parametrize("hq", [2, 32])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("large,top", [((10, 11), 100), ((1000, 1001), 5)])
+def test_values_whose_sum_overflows_only_without_the_row_maximum(hq, d, large, top):
+    # two values of 3e38 at keys e^-8 below the row's largest, which lies in another
+    # tile of their block or in another chunk: the result is finite
+    S = 1500
+    q = torch.zeros(S, hq, d, device=DEV)
+    k, v = torch.zeros(S, 1, d, device=DEV), torch.zeros(S, 1, d, device=DEV)
+    q[..., 0] = math.sqrt(d)
+    k[:, 0, 0] = -1000.0
+    k[list(large), 0, 0] = 0.0
+    k[top, 0, 0] = 8.0
+    v[list(large), 0, 5] = 3e38
+    got = _run(q, k, v, 128, 100)[1002:, :, 5].double()
+    want = 6e38 * math.exp(-8) / (1 + 2 * math.exp(-8))
+    assert ((got - want) / want).abs().max().item() <= 9 * 8 * 2.0 ** -24
