@@ -369,6 +369,65 @@ __global__ __launch_bounds__(256, D > 128 ? 2 : 3) void k_paged(PagedArgs a) {
     if (more) load_v_tiles(next);
   }
 
+  // O not finite: P.V again over the keys that each row sees (a masked key's infinite
+  // or NaN value times P = 0 is NaN), with P and l 2^off times smaller (m larger), so
+  // that values near the largest do not overflow before the division by l
+  {
+    float nf = 0.0f;
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) nf = fmaf(acc[e][v], 0.0f, nf);
+    if (__ballot(nf != 0.0f) != 0) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) acc[e] = f32x4{};
+      const float off = static_cast<float>(32 - __clz(k1 - k0));
+      m_run += off;
+      l_part *= __builtin_amdgcn_exp2f(-off);
+      const float ms = m_run == -INFINITY ? 0.0f : m_run;
+      int lane2 = static_cast<int>(threadIdx.x);  // (formed here, not kept across the loop)
+      asm volatile("" : "+v"(lane2));
+      const int g2 = (lane2 >> 4) & 3;
+#pragma unroll 1
+      for (int i = 0; i < 32 * ((k1 - k0 + 127) / 128); ++i) {
+        const int key = k0 + 32 * w + 128 * (i >> 5) + (i & 31);
+        if (key >= k1) break;
+        const int64_t pg = paged_page<true>(a, row, key, bad);
+        const int in = key % a.bs;
+        const uint16_t* kp = kc + pg * a.kcb + static_cast<int64_t>(in) * a.kcs + 8 * g2;
+        const uint16_t* vp = vc + pg * a.vcb + static_cast<int64_t>(in) * a.vcs;
+        float x = 0.0f;  // the lane's dims of q . k
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          const uint4 ku = ld16(kp + 32 * ks), qu = __builtin_bit_cast(uint4, qb[ks]);
+          const uint32_t kw[4] = {ku.x, ku.y, ku.z, ku.w}, qw[4] = {qu.x, qu.y, qu.z, qu.w};
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            x = fmaf(T::to_f32(static_cast<uint16_t>(qw[e])),
+                     T::to_f32(static_cast<uint16_t>(kw[e])), x);
+            x = fmaf(T::to_f32(static_cast<uint16_t>(qw[e] >> 16)),
+                     T::to_f32(static_cast<uint16_t>(kw[e] >> 16)), x);
+          }
+        }
+        x = row4_sum(x) * scale;
+        if (key > lim) continue;
+        const float p = __builtin_amdgcn_exp2f(x - ms);
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+          for (int e = 0; e < E; e += 4) {
+            const int dim = D == 64 ? 4 * (4 * g2 + v)
+                                    : 128 * (e >> 3) + 8 * (4 * g2 + v) + (e & 7);
+            const uint2 u = *reinterpret_cast<const uint2*>(vp + dim);
+            acc[e][v] = fmaf(p, T::to_f32(static_cast<uint16_t>(u.x)), acc[e][v]);
+            acc[e + 1][v] = fmaf(p, T::to_f32(static_cast<uint16_t>(u.x >> 16)), acc[e + 1][v]);
+            acc[e + 2][v] = fmaf(p, T::to_f32(static_cast<uint16_t>(u.y)), acc[e + 2][v]);
+            acc[e + 3][v] = fmaf(p, T::to_f32(static_cast<uint16_t>(u.y >> 16)), acc[e + 3][v]);
+          }
+      }
+    }
+  }
+
   // acc[e][v] is dim 8 (4 g + v) + e (+ 120 per e >= 8 at d = 256: the second
   // 128 dims), d = 64: dim 4 (4 g + v) + e, of row r16
   float l = row4_sum(l_part);
@@ -399,7 +458,8 @@ __global__ __launch_bounds__(256, D > 128 ? 2 : 3) void k_paged(PagedArgs a) {
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     const float mk = sml[k][orow][0];
-    const float f = mk == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mk - M);
+    // (a quarter each: four finite sums add up to a finite one)
+    const float f = mk == -INFINITY ? 0.0f : 0.25f * __builtin_amdgcn_exp2f(mk - M);
     // (a wave without keys has m = -inf and l = 0; NaN scores leave m = -inf
     // with l = NaN, which the sum keeps)
     L += mk == -INFINITY ? sml[k][orow][1] : f * sml[k][orow][1];
@@ -460,8 +520,9 @@ __global__ __launch_bounds__(256) void k_paged_merge(PagedArgs a) {
     l1 = a.ml[2 * (slot + lane + 64) + 1];
   }
   const float M = wave_max(fmaxf(m0, m1));
-  const float f0 = m0 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m0 - M);
-  const float f1 = m1 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m1 - M);
+  // (2^-7: the sum over at most 128 chunks stays finite)
+  const float f0 = m0 == -INFINITY ? 0.0f : 0x1p-7f * __builtin_amdgcn_exp2f(m0 - M);
+  const float f1 = m1 == -INFINITY ? 0.0f : 0x1p-7f * __builtin_amdgcn_exp2f(m1 - M);
   float L = (m0 == -INFINITY ? l0 : f0 * l0) + (m1 == -INFINITY ? l1 : f1 * l1);
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) L += __shfl_xor(L, o);
@@ -775,8 +836,9 @@ __global__ __launch_bounds__(256, 2) void k_paged_rows(PagedArgs a) {
   }
 
   // An infinite or NaN value times the parts of P is NaN where its product with P
-  // is not (a part may be 0 or negative), so rows whose O is not finite take P.V
-  // again in fp32 with P whole, over the keys that each row sees; m and l hold.
+  // is not (a part may be 0 or negative), and sums of values near the largest
+  // overflow before they are divided by l: rows whose O is not finite take P.V again
+  // in fp32 with P whole, over the keys that each row sees.
   float nf = 0.0f;
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
@@ -785,6 +847,11 @@ __global__ __launch_bounds__(256, 2) void k_paged_rows(PagedArgs a) {
   if (__ballot(nf != 0.0f) != 0) {
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) o[dt] = f32x16{};
+    // P and l 2^off times smaller (m larger): the sum of P V then stays below the
+    // largest value, as that of normalised weights does
+    const float off = static_cast<float>(32 - __clz(k1 - k0));
+    m_run += off;
+    l_part *= __builtin_amdgcn_exp2f(-off);
     const float ms = (m_run == -INFINITY ? 0.0f : m_run) - PParts<T>::kPShift;
     // (formed here: kept live across the loop above, the offsets cost d = 64 its
     // third wave per SIMD, 781 -> 826 us for 4 x 2,048 new of 6,144 tokens)
@@ -906,7 +973,7 @@ __global__ __launch_bounds__(256) void k_paged_merge_rows(PagedArgs a) {
 #pragma unroll
     for (int u = 0; u < H; ++u) {
       const float m = a.ml[2 * (slot[u] + c)], l = a.ml[2 * (slot[u] + c) + 1];
-      const float f = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - M[u]);
+      const float f = m == -INFINITY ? 0.0f : 0x1p-7f * __builtin_amdgcn_exp2f(m - M[u]);
       L[u] += m == -INFINITY ? l : f * l;
 #pragma unroll
       for (int q = 0; q < XD; ++q) acc[u][q] += f * a.part[(slot[u] + c) * D + XD * lane + q];

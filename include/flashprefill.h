@@ -215,6 +215,7 @@ int fp_kv_cache_write(const fp_kv_cache_args* a, void* stream);
  * has room for make the sequence's rows NaN, a page number outside the cache the
  * rows that attend to it; a row with no cached token to attend to is NaN, a
  * sequence of no cached tokens 0.
+ * An infinite or NaN value reaches the rows that attend to its key only.
  * Strides in elements (multiples of 8, 16-byte aligned bases), head dim
  * contiguous. The integer arrays hold 32- or 64-bit integers. */
 typedef struct fp_paged_args {

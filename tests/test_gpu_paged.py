@@ -285,16 +285,33 @@ def test_infinite_values(dtype, news, d, page):
 
 
 @pytest.mark.parametrize("value", [math.inf, math.nan])
-def test_a_value_that_a_row_does_not_see(value):
-    """At many rows per sequence: an infinity or NaN in V at the last new token
-    reaches the last query only, the rows before it stay finite."""
-    args = _case([500], [40], 8, 2, 128, 16, torch.bfloat16, seed=4)
+@pytest.mark.parametrize("news,d", [(40, 128), (3, 128), (3, 64), (3, 256)])
+def test_a_value_that_a_row_does_not_see(value, news, d):
+    """An infinity or NaN in V at the last new token reaches the last query only,
+    the rows before it stay finite."""
+    args = _case([500], [news], 8, 2, d, 16, torch.bfloat16, seed=4)
     want = _want(*args, 0.1)
     args[2][args[5][0, 499 // 16], 499 % 16, :, 7] = value
     got = _run(args, 0.1).double()
-    assert torch.equal(got[39, :, 7].isnan(), torch.full((8,), math.isnan(value)))
-    assert not got[39, :, 7].isfinite().any()
-    assert ((got - want).abs()[:39] <= want.abs()[:39] * 2.0 ** -8 * 1.01 + 2e-6).all()
+    last = news - 1
+    assert torch.equal(got[last, :, 7].isnan(), torch.full((8,), math.isnan(value)))
+    assert not got[last, :, 7].isfinite().any()
+    bound = want.abs()[:last] * 2.0 ** -8 * 1.01 + 2e-6
+    assert ((got - want).abs()[:last] <= bound).all()
+
+
+@pytest.mark.parametrize("news", [1, 40])
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("page", [16, 24])
+def test_values_near_the_largest(news, d, page):
+    """V of 3.3e38 at every key of a dim: the weighted mean is that value, whatever
+    the sum of the weights before the division, in one chunk and in several."""
+    args = _case([3000, 200], [news] * 2, 8, 2, d, page, torch.bfloat16, seed=5)
+    args[2][:, :, 0, 3] = 3.3e38
+    args[2][:, :, 1, d - 2] = -3.3e38
+    got, want = _run(args, 0.05).double(), _want(*args, 0.05)
+    assert want.isfinite().all()
+    assert ((got - want).abs() <= want.abs() * 2.0 ** -8 * 1.01 + 2e-6).all()
 
 
 @pytest.mark.parametrize("d", [64, 128])
